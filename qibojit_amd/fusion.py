@@ -92,6 +92,31 @@ def fused_matrix(custom_matrix_of, fgate):
     return m
 
 
+def channel_superoperator(custom_matrix_of, channel, block):
+    """4^k x 4^k matrix of rho -> sum_i c_i K_i rho K_i^+ + (1 - sum c) rho on
+    the k row bits and then the k column bits of ``block`` (sorted qubits).
+
+    Entry [(a, c), (b, d)] is sum_i c_i K_i[a, b] conj(K_i[c, d]).  The terms
+    of a channel of unitaries need invertible operators (the operator sum
+    undoes each one before the next), so a singular one raises
+    ``LinAlgError`` here as it does there."""
+    dim = 2 ** len(block)
+    pairs = list(zip(channel.coefficients, channel.gates))
+    ks = np.empty((len(pairs), dim, dim), dtype=complex)
+    for i, (_, gate) in enumerate(pairs):
+        u = target_block(custom_matrix_of, gate)
+        whole = len(gate.control_qubits) == 0 and list(gate.target_qubits) == block
+        ks[i] = u if whole else embed(block, gate.target_qubits, gate.control_qubits, u)
+    if channel._all_unitary_operators:  # pylint: disable=protected-access
+        np.linalg.inv(ks)
+    coeffs = np.asarray([c for c, _ in pairs], dtype=complex)
+    flat = ks.reshape(len(ks), -1)
+    terms = (flat * coeffs[:, None]).T @ flat.conj()  # [(a, b), (c, d)]
+    out = terms.reshape((dim,) * 4).transpose(0, 2, 1, 3).reshape(dim * dim, dim * dim)
+    out.flat[:: dim * dim + 1] += 1 - channel.coefficient_sum
+    return out
+
+
 def plan_blocks(gate_qubits, max_qubits=5):
     """Group a gate sequence into blocks of at most ``max_qubits`` qubits.
 
