@@ -352,6 +352,195 @@ __global__ void __launch_bounds__(kRotBlock)
   if (threadIdx.x == 0) partials[(u64)b * gridDim.x + blockIdx.x] = acc;
 }
 
+// Energies from tiles.  k_tfim_batch reads a partner group per flip; here a
+// workgroup holds a 64 KiB tile of the state (after the ladder: the
+// permutation is taken while loading) and every flip inside the tile is a
+// pair of registers: a thread holds 16 amplitudes, four tile bits, and reads
+// them anew from LDS for the next four, so a flip costs one multiply-add per
+// component and pair and nothing is exchanged.  A launch covers the bits in
+// passes (the low TB bits, then a low run of whole lines plus the next
+// TB - L bits each), one read of the state per pass; a pass's tiles go to
+// `cols` of the launch's workgroups, which load the next tile into registers
+// while they work on the current one.  Bound by the reads of the state above
+// the caches (26 qubits complex128, 3 passes: 0.50 ms, 6.5 TB/s; the former
+// kernel of single states read the partners from memory, 2.28 ms) and by the
+// conversions to FP64 for complex64 batches in them (16 states of 22 qubits:
+// 0.51 -> 0.27 ms against k_tfim_batch on a full grid; complex128 0.86 -> 0.49).
+constexpr int kTfimMaxPasses = 6;
+struct TfimPass {
+  int L;             // low run of the tile
+  int h0;            // first bit of its high part
+  unsigned active;   // tile bits whose flips the pass takes
+};
+struct TfimTiles {
+  int npass;
+  int cols;          // workgroups per pass
+  TfimPass pass[kTfimMaxPasses];
+};
+
+// LDS slot of tile element e: the four bits a wave strides over in the layout
+// with the lowest register bits are folded into its bank bits.
+template <int TB>
+__device__ __forceinline__ unsigned tfim_slot(unsigned e) {
+  return TB == 13 ? e ^ (((e >> 5) & 15u) << 1) : e ^ ((e >> 4) & 15u);
+}
+
+// Adds Re(conj(x) y) of the pairs of the active flips of register bits S..S+3.
+template <typename R, int TB, int S>
+__device__ __forceinline__ double tfim_flips(const cplx<R>* tile, int t, unsigned active) {
+  if (!((active >> S) & 15u)) return 0.0;  // uniform
+  const unsigned te = (unsigned)((t & ((1 << S) - 1)) | ((t >> S) << (S + 4)));
+  unsigned ts = tfim_slot<TB>(te);
+  asm volatile("" : "+v"(ts));  // keeps the 16 addresses out of the tile loop's live registers
+  double re[16], im[16], xs = 0.0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const cplx<R> v = tile[ts ^ tfim_slot<TB>((unsigned)j << S)];
+    re[j] = v.re;
+    im[j] = v.im;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if ((active >> (S + r)) & 1u)  // uniform
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (!((j >> r) & 1)) xs += re[j] * re[j | (1 << r)] + im[j] * im[j | (1 << r)];
+  return xs;
+}
+
+template <typename R, int TB>
+__global__ void __launch_bounds__(1 << (TB - 4), TB == 13 ? 4 : 2)
+    k_tfim_tile(const cplx<R>* __restrict__ psi, const int32_t* __restrict__ sel, u64 stride, int nq, double g,
+                int ladder, TfimTiles tt, int ncols, double* __restrict__ partials) {
+  constexpr int TBITS = TB - 4, NT = 1 << TBITS;
+  __shared__ cplx<R> tile[1 << TB];
+  __shared__ double wsum[NT / 64];
+  const int b = blockIdx.y, pi = (int)blockIdx.x / tt.cols;
+  double acc = 0.0;
+  {
+    const TfimPass ps = tt.pass[pi];
+    const cplx<R>* p = psi + (sel ? (u64)sel[b] : (u64)b) * stride;
+    const u64 zzmask = (u64(1) << (nq - 1)) - 1;
+    const int t = (int)threadIdx.x;
+    const u64 lowmask = (u64(1) << ps.L) - 1;
+    // tile element e -> offset of its amplitude from the tile's base
+    auto spread = [&](unsigned e) { return ((u64)(e >> ps.L) << ps.h0) | (e & lowmask); };
+    const u64 toff = spread((unsigned)t);
+    // tile number -> base: bits L..h0-1 and the bits above the high part
+    const int mid = ps.h0 - ps.L;
+    auto base_of = [&](u64 tau) {
+      return ((tau & ((u64(1) << mid) - 1)) << ps.L) | ((tau >> mid) << (ps.h0 + TB - ps.L));
+    };
+    // amplitude k after the ladder is k ^ (k >> 1) before it (linear in k)
+    auto source = [&](u64 k) { return ladder ? k ^ (k >> 1) : k; };
+    const u64 ntiles = u64(1) << (nq - TB);
+    cplx<R> x[16];
+    u64 tau = (u64)((int)blockIdx.x % tt.cols);
+    if (tau < ntiles) {
+      const u64 base = source(base_of(tau) | toff);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j] = p[base ^ source(spread((unsigned)j << TBITS))];
+    }
+    for (; tau < ntiles; tau += (u64)tt.cols) {  // uniform
+      __syncthreads();  // the former tile's reads are done
+      unsigned ts = tfim_slot<TB>((unsigned)t);
+      asm volatile("" : "+v"(ts));
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        tile[ts ^ tfim_slot<TB>((unsigned)j << TBITS)] = x[j];
+      if (pi == 0) {
+        const u64 base = base_of(tau) | toff;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const u64 k = base | spread((unsigned)j << TBITS);
+          const double zz = (double)(nq - 1 - 2 * (int)__popcll((k ^ (k >> 1)) & zzmask));
+          const double xr = x[j].re, xi = x[j].im;
+          acc -= zz * (xr * xr + xi * xi);
+        }
+      }
+      const u64 next = tau + (u64)tt.cols;
+      if (next < ntiles) {
+        const u64 base = source(base_of(next) | toff);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[j] = p[base ^ source(spread((unsigned)j << TBITS))];
+      }
+      __syncthreads();
+      // one layout's amplitudes live at a time: the scheduler would otherwise
+      // read the next layout's ahead and spill
+      __builtin_amdgcn_sched_barrier(0);
+      double xs = tfim_flips<R, TB, TB - 4>(tile, t, ps.active);
+      __builtin_amdgcn_sched_barrier(0);
+      xs += tfim_flips<R, TB, TB - 8>(tile, t, ps.active);
+      __builtin_amdgcn_sched_barrier(0);
+      xs += tfim_flips<R, TB, TB - 12>(tile, t, ps.active);
+      __builtin_amdgcn_sched_barrier(0);
+      if (TB == 13) xs += tfim_flips<R, TB, 0>(tile, t, ps.active & 1u);
+      acc -= 2.0 * g * xs;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double sum = 0.0;
+    for (int w = 0; w < NT / 64; ++w) sum += wsum[w];
+    partials[(u64)b * ncols + blockIdx.x] = sum;
+  }
+  if (blockIdx.x == 0)  // columns without a workgroup
+    for (int c = (int)gridDim.x + (int)threadIdx.x; c < ncols; c += NT) partials[(u64)b * ncols + c] = 0.0;
+}
+
+// Passes over nq bits with tiles of tb bits: the first takes bits 0..tb-1,
+// every later one keeps a low run of 4 bits (128 bytes complex64; 256 bytes
+// complex128, 3 bits where that saves a pass) and takes the next bits.
+static TfimTiles tfim_tiles(int nq, int tb, bool c64) {
+  auto passes = [&](int run) { return 1 + (nq - tb + tb - run - 1) / (tb - run); };
+  const int run = !c64 && passes(3) < passes(4) ? 3 : 4;
+  TfimTiles tt;
+  std::memset(&tt, 0, sizeof(tt));
+  tt.pass[0] = {tb, tb, (1u << tb) - 1};
+  tt.npass = 1;
+  for (int q = tb; q < nq; ++tt.npass) {
+    const int h = std::min(nq - q, tb - run);
+    tt.pass[tt.npass] = {tb - h, q, ((1u << h) - 1) << (tb - h)};
+    q += h;
+  }
+  return tt;
+}
+
+// Rows and tiles that are worth a tile launch: below, k_tfim_batch's smaller
+// workgroups spread better (one 16-qubit complex64 state, 8 tiles: 30.3
+// against 27.2 us with the readback; 64 states of 13 qubits: 7.9 against 20.9).
+constexpr u64 kTfimMinTiles = 64;
+// Workgroups of a launch: the resident ones twice over.
+constexpr u64 kTfimTileBlocks = 1024;
+constexpr u64 kTfimNarrow = u64(1) << 18;
+
+// Launches k_tfim_tile for rows of ncols partials; 0 if the rows have too few
+// tiles or partials.
+static int launch_tfim_tile(const void* psi, int dtype, int nq, u64 stride, const int32_t* sel, int nrows, double g,
+                            int ladder, double* partials, int ncols, hipStream_t st) {
+  const bool c64 = dtype == QJ_COMPLEX64;
+  if (!c64 && dtype != QJ_COMPLEX128) return 0;
+  const int tb = c64 ? 13 : 12;
+  if (nq < tb) return 0;
+  const u64 ntiles = u64(1) << (nq - tb);
+  if (ntiles * (u64)nrows < kTfimMinTiles) return 0;
+  TfimTiles tt = tfim_tiles(nq, tb, c64);
+  const u64 want = std::max<u64>(1, kTfimTileBlocks / ((u64)nrows * tt.npass));
+  tt.cols = (int)std::min<u64>(std::min(ntiles, want), ncols / tt.npass);
+  if (tt.cols < 1) return 0;
+  const dim3 gd((unsigned)(tt.cols * tt.npass), (unsigned)nrows);
+  if (c64)
+    k_tfim_tile<float, 13><<<gd, dim3(512), 0, st>>>((const cplx<float>*)psi, sel, stride, nq, g, ladder, tt, ncols,
+                                                     partials);
+  else
+    k_tfim_tile<double, 12><<<gd, dim3(256), 0, st>>>((const cplx<double>*)psi, sel, stride, nq, g, ladder, tt, ncols,
+                                                     partials);
+  return 1;
+}
+
 // out[r] = sum_c in[r * ncols + c], one workgroup per row, fixed order.
 __global__ void __launch_bounds__(kRotBlock) k_reduce_rows(const double* __restrict__ in, u64 ncols,
                                                            double* __restrict__ out) {
@@ -965,10 +1154,14 @@ int qj_tfim_batch(const void* psi, void* out, int dtype, int nqubits, uint64_t s
   if (psi == out) return set_error(QJ_EVALUE, "tfim_batch: out must not alias psi");
   hipStream_t st = (hipStream_t)stream;
   dim3 gd((unsigned)ncols, (unsigned)nrows);
+  if (!out && launch_tfim_tile(psi, dtype, nqubits, stride, sel, nrows, g, ladder, partials, ncols, st))
+    return check_launch("tfim_batch launch");
   // vector groups of 32 bytes when every state starts on one (the state
-  // pointers are at least 256-byte aligned)
+  // pointers are at least 256-byte aligned); a launch of few amplitudes keeps
+  // one per thread, which spreads it over more CUs
+  const bool wide = ((u64)nrows << nqubits) > kTfimNarrow;
   if (dtype == QJ_COMPLEX64) {
-    if (stride % 4 == 0 && (reinterpret_cast<uintptr_t>(psi) & 31) == 0 &&
+    if (wide && stride % 4 == 0 && (reinterpret_cast<uintptr_t>(psi) & 31) == 0 &&
         (!out || (reinterpret_cast<uintptr_t>(out) & 31) == 0))
       k_tfim_batch<float, 4><<<gd, dim3(kRotBlock), 0, st>>>((const cplx<float>*)psi, (cplx<float>*)out, sel,
                                                              stride, nqubits, g, ladder != 0, partials);
@@ -976,7 +1169,7 @@ int qj_tfim_batch(const void* psi, void* out, int dtype, int nqubits, uint64_t s
       k_tfim_batch<float, 1><<<gd, dim3(kRotBlock), 0, st>>>((const cplx<float>*)psi, (cplx<float>*)out, sel,
                                                              stride, nqubits, g, ladder != 0, partials);
   } else if (dtype == QJ_COMPLEX128) {
-    if (stride % 2 == 0 && (reinterpret_cast<uintptr_t>(psi) & 31) == 0 &&
+    if (wide && stride % 2 == 0 && (reinterpret_cast<uintptr_t>(psi) & 31) == 0 &&
         (!out || (reinterpret_cast<uintptr_t>(out) & 31) == 0))
       k_tfim_batch<double, 2><<<gd, dim3(kRotBlock), 0, st>>>((const cplx<double>*)psi, (cplx<double>*)out, sel,
                                                               stride, nqubits, g, ladder != 0, partials);

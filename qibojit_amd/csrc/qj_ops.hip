@@ -648,36 +648,6 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// <psi|H|psi>, H = -sum Z_i Z_{i+1} - g sum X_i on an open chain of n qubits.
-// Diagonal: sum_i z_i z_{i+1} = (n-1) - 2 popcount((k ^ (k >> 1)) & (2^(n-1)-1)).
-// X_b term: sum_k Re(conj(psi_k) psi_{k^2^b}) = 2 sum_{bit b of k = 0} Re(...).
-template <typename R>
-__global__ void __launch_bounds__(kBlock)
-    k_tfim(const cplx<R>* __restrict__ st, int nq, double g, double* __restrict__ partials) {
-  __shared__ double wsum[kBlock / 64];
-  const u64 n = u64(1) << nq;
-  const u64 zzmask = (u64(1) << (nq - 1)) - 1;
-  double acc = 0.0;
-  const u64 stride = (u64)gridDim.x * kBlock;
-  for (u64 k = (u64)blockIdx.x * kBlock + threadIdx.x; k < n; k += stride) {
-    const cplx<R> x = st[k];
-    const int pc = __popcll((k ^ (k >> 1)) & zzmask);
-    const double zz = (double)(nq - 1) - 2.0 * (double)pc;
-    acc -= zz * abs2(x);
-    double xs = 0.0;
-    for (int b = 0; b < nq; ++b) {
-      const u64 bit = u64(1) << b;
-      if (!(k & bit)) {
-        const cplx<R> y = st[k | bit];
-        xs += (double)x.re * (double)y.re + (double)x.im * (double)y.im;
-      }
-    }
-    acc -= 2.0 * g * xs;
-  }
-  acc = block_sum(acc, wsum);
-  if (threadIdx.x == 0) partials[blockIdx.x] = acc;
-}
-
 template <typename R>
 __global__ void __launch_bounds__(kBlock)
     k_axpby(const cplx<R>* __restrict__ x, cplx<R>* __restrict__ y, u64 n, cplx<R> a, cplx<R> b) {
@@ -1434,15 +1404,10 @@ int qj_expectation_tfim(const void* state, int dtype, int nqubits, double g, dou
   DeviceScratch* sc = nullptr;
   int rc = scratch_for_current_device(&sc);
   if (rc) return rc;
-  const u64 n = u64(1) << nqubits;
-  const u64 grid = std::min<u64>(kRedBlocks, grid_for(n, kBlock));
-  if (dtype == QJ_COMPLEX64)
-    k_tfim<float><<<dim3((unsigned)grid), dim3(kBlock), 0, s>>>((const cplx<float>*)state, nqubits, g, sc->partials);
-  else if (dtype == QJ_COMPLEX128)
-    k_tfim<double><<<dim3((unsigned)grid), dim3(kBlock), 0, s>>>((const cplx<double>*)state, nqubits, g, sc->partials);
-  else
-    return set_error(QJ_EVALUE, "expectation_tfim: dtype must be complex");
-  rc = check_launch("tfim launch");
+  // one row of the batched kernels
+  const u64 grid = std::min<u64>(kRedBlocks, grid_for(u64(1) << nqubits, kBlock));
+  rc = qj_tfim_batch(state, nullptr, dtype, nqubits, u64(1) << nqubits, nullptr, 1, g, 0, sc->partials, (int)grid,
+                     stream);
   if (rc) return rc;
   return reduce_to_host(1, grid, 0, 1, out, s, sc);
 }
