@@ -487,10 +487,21 @@ int qj_clifford_determined_outcome_exact(uint32_t* tab, int nqubits, int q, int3
  * random outcomes taken before it), a determined one the reference's XOR
  * rule (exact != 0: the rule of qj_clifford_determined_outcome_exact).
  * sample_out (device int32, m) gets the outcomes, *nrandom_out (device
- * int32) the number of random ones.  Same tableau and outcomes as the
+ * int32) the number of random ones, or -1 if the device loop gave up waiting
+ * (the tableau is then undefined).  Same tableau and outcomes as the
  * per-qubit entry points. */
 int qj_clifford_measure(uint32_t* tab, int nqubits, const int32_t* qubits, int m, const uint8_t* draws, int exact,
                         int32_t* sample_out, int32_t* nrandom_out, void* stream);
+/* The affine forms of the outcomes of qj_clifford_measure (exact == 0) in the
+ * random ones, in one pass that leaves the tableau unchanged: row i of
+ * `forms` (device uint8, m x (m + 1), zeroed by the caller) holds the constant
+ * term and the coefficients of the random outcomes u_1..u_k of outcome i,
+ * *nrandom_out (device int32) is k.  Tableaux whose rows do not fit the LDS
+ * of one resident workgroup per 32 rows, and streams under capture, get
+ * QJ_EVALUE (qj_clifford_forms_supported(nqubits, m) == 0 for the former). */
+int qj_clifford_forms_supported(int nqubits, int m);
+int qj_clifford_measurement_forms(const uint32_t* tab, int nqubits, const int32_t* qubits, int m, uint8_t* forms,
+                                  int32_t* nrandom_out, void* stream);
 /* rowsum of clifford_operations_cpu.py:337-385 on host arrays h, i of
  * nrows row indices: row h[j] <- P_{i[j]} P_{h[j]} (x, z XORed; r = (2 r_h +
  * 2 r_i + sum of the exponents of i) mod 4 != 0), every product from the

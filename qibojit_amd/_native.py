@@ -78,6 +78,7 @@ SIGNATURES = {
     "qj_clifford_determined_outcome": [_vp, _i32, _i32, _vp, _vp],
     "qj_clifford_determined_outcome_exact": [_vp, _i32, _i32, _vp, _vp],
     "qj_clifford_measure": [_vp, _i32, _vp, _i32, _vp, _i32, _vp, _vp, _vp],
+    "qj_clifford_measurement_forms": [_vp, _i32, _pi32, _i32, _vp, _vp, _vp],
     "qj_clifford_rowsum": [_vp, _i32, _vp, _vp, _i64, _i32, _vp],
     "qj_clifford_sym_init": [_vp, _i32, _vp, _i32, _vp],
     "qj_clifford_sym_random": [_vp, _i32, _vp, _i32, _i32, _i32, _i32, _vp],
@@ -91,6 +92,7 @@ SIGNATURES = {
 # entry points that return a value instead of a status
 VALUE_SIGNATURES = {
     "qj_clifford_column_words": (ctypes.c_int64, [_i32]),
+    "qj_clifford_forms_supported": (ctypes.c_int, [_i32, _i32]),
 }
 
 _LIB = None

@@ -297,6 +297,8 @@ def M(state, qubits, nqubits, collapse=False, exact=False):
                  _ptr(draws_d), int(bool(exact)), _ptr(out), _ptr(out[m:]), _stream(state))
     host = out.cpu().numpy()
     np.random.set_state(saved)
+    if host[m] < 0:
+        raise RuntimeError("the device measurement loop did not finish")
     np.random.randint(2, size=int(host[m]), dtype=np.uint)
     return [int(v) for v in host[:m]]
 
@@ -337,6 +339,16 @@ def measurement_forms(state, qubits, nqubits, exact=False):
     _check_tableau(state, nqubits)
     qubits = [int(q) for q in qubits]
     m, n = len(qubits), int(nqubits)
+    if m and not exact and _native.lib().qj_clifford_forms_supported(n, m) \
+            and not torch.cuda.is_current_stream_capturing():
+        buf = torch.zeros(4 + m * (m + 1), dtype=torch.uint8, device=state.device)
+        qs = (ctypes.c_int32 * m)(*qubits)
+        _native.call("qj_clifford_measurement_forms", _ptr(state), n, qs, m, _ptr(buf[4:]), _ptr(buf), _stream(state))
+        host = buf.cpu().numpy()
+        k = int(host[:4].view(np.int32)[0])
+        if k < 0:
+            raise RuntimeError("the device measurement loop did not finish")
+        return np.ascontiguousarray(host[4:].reshape(m, m + 1)[:, : k + 1]), k
     tab = state.clone()
     signs = torch.empty(((m + 1), column_words(n)), dtype=torch.int32, device=state.device)
     forms = torch.zeros((m, m + 1), dtype=torch.uint8, device=state.device)

@@ -777,6 +777,8 @@ __global__ __launch_bounds__(1024) void k_cliff_measure_small(uint32_t* __restri
   if (tid == 0) nrandom[0] = count;
 }
 
+#include "qj_cliff_rows.h"
+
 // ---- general rowsum (clifford_operations_cpu.py:337-385) ----
 
 // New sign of every pair from the state before the call: rnew[j], and
@@ -1422,6 +1424,92 @@ void launch_circuit(uint32_t* tab, int nqubits, const uint32_t* ddesc, int64_t n
   }
 }
 
+// Shape of k_cliff_measure_rows for n qubits and S sign columns: one workgroup
+// up to 256 qubits (no exchange), else 32 rows each, so that every workgroup
+// is resident and its slice fits LDS.
+struct RowsPlan {
+  int R, G, dw;
+  size_t lds;
+};
+bool rows_plan(int n, int S, RowsPlan* p) {
+  const int nw = (n + 31) / 32;
+  int cus = 0;
+  size_t max_lds = 0;
+  device_lds(&cus, &max_lds);
+  p->R = 1;
+  if (nw <= 8)
+    while (p->R < nw) p->R *= 2;
+  else if (const char* e = std::getenv("QJ_RT")) p->R = std::atoi(e);
+  p->G = (nw + p->R - 1) / p->R;
+  const int64_t C = 2 * (int64_t)n + S;
+  p->dw = (int)(2 * ((C + 63) / 64));
+  p->lds = ((size_t)2 * C * p->R + 2 * (size_t)p->dw) * sizeof(uint32_t);
+  const size_t cap = std::min(kCliffLdsPerCu, std::max<size_t>(max_lds, 65536)) - 2048;  // static part
+  return p->G <= cus && p->G <= 256 && p->lds <= cap;
+}
+
+template <bool SYM>
+const void* rows_kernel(int R) {
+  switch (R) {
+    case 1: return reinterpret_cast<const void*>(&k_cliff_measure_rows<1, SYM>);
+    case 2: return reinterpret_cast<const void*>(&k_cliff_measure_rows<2, SYM>);
+    case 4: return reinterpret_cast<const void*>(&k_cliff_measure_rows<4, SYM>);
+    default: return reinterpret_cast<const void*>(&k_cliff_measure_rows<8, SYM>);
+  }
+}
+
+// Runs the measurement loop of a.m qubits in one launch; 0 if this tableau or
+// stream (one under capture) is not for it, else 1 with the status in *rc.
+template <bool SYM>
+int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStream_t s, int* rc) {
+  RowsPlan p;
+  if (!rows_plan(a.n, a.S, &p)) return 0;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  const int64_t W = cliff_words(a.n), C = 2 * (int64_t)a.n + 1;
+  const size_t posts = (size_t)2 * p.G * (1 + p.dw);
+  const size_t stage = SYM ? 0 : (size_t)2 * C * p.G * p.R, scratch = SYM ? 0 : (size_t)p.G * (p.dw + 1);
+  DeviceScratch* sc = nullptr;
+  *rc = scratch_for_current_device(&sc);
+  if (*rc) return 1;
+  *rc = scratch_reserve_big(sc, posts * sizeof(post_t) + (stage + scratch + 4) * sizeof(uint32_t), s);
+  if (*rc) return 1;
+  a.tab = tab;
+  a.ws = cliff_stride(a.n);
+  a.dw = p.dw;
+  a.hdr = static_cast<post_t*>(sc->big);
+  a.data = a.hdr + (size_t)2 * p.G;
+  a.stage = reinterpret_cast<uint32_t*>(a.hdr + posts);
+  a.scratch = a.stage + stage;
+  a.det_any = reinterpret_cast<int32_t*>(a.scratch + scratch);
+  void* dq = nullptr;
+  int ticket = -1;
+  *rc = ring_upload(qubits, (size_t)a.m * sizeof(int32_t), s, &dq, &ticket);
+  if (*rc) return 1;
+  a.qubits = static_cast<const int32_t*>(dq);
+  const void* kern = rows_kernel<SYM>(p.R);
+  if (p.lds > 65536) (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
+  void* args[] = {&a};
+  if (p.G == 1) {
+    *rc = hip_status(hipLaunchKernel(kern, dim3(1), dim3(kRowsThreads), args, p.lds, s), "clifford_measure launch");
+  } else {
+    // no word of an earlier launch may carry a step of this one
+    k_fill_words<<<dim3(blocks_for((int64_t)posts * 2, kBlock)), dim3(kBlock), 0, s>>>(
+        reinterpret_cast<uint32_t*>(a.hdr), (int64_t)posts * 2, 0u);
+    *rc = hip_status(hipLaunchCooperativeKernel(kern, dim3((unsigned)p.G), dim3(kRowsThreads), args,
+                                                (unsigned)p.lds, s), "clifford_measure cooperative launch");
+  }
+  if (!*rc && !SYM) {
+    k_cliff_merge_rows<<<dim3(blocks_for(C * W, kBlock)), dim3(kBlock), 0, s>>>(tab, a.n, a.ws, W, a, p.G, p.R);
+    *rc = check_launch("clifford_measure merge launch");
+  }
+  ring_release(ticket, s);
+  return 1;
+}
+
 }  // namespace
 }  // namespace qj
 
@@ -1611,6 +1699,17 @@ int qj_clifford_measure(uint32_t* tab, int nqubits, const int32_t* qubits, int m
   const char* mode = std::getenv("QJ_CLIFFORD_MEASURE");
   const bool force_kernels = mode && std::strcmp(mode, "kernels") == 0;
   const bool force_small = mode && std::strcmp(mode, "small") == 0;
+  if (!exact && !force_kernels && !force_small) {
+    RowsArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.n = nqubits;
+    a.m = m;
+    a.S = 1;
+    a.draws = draws;
+    a.sample = sample_out;
+    a.nrandom = nrandom_out;
+    if (launch_measure_rows<false>(tab, a, qubits, s, &rc)) return rc;
+  }
   if (!force_kernels && (nqubits <= kMeasureSmallMax || (force_small && nqubits <= kMeasureSmallCap))) {
     void* dq = nullptr;
     int ticket = -1;
@@ -1712,6 +1811,32 @@ int qj_clifford_rowsum(uint32_t* tab, int nqubits, const int64_t* h, const int64
                                                                                     flip);
   rc = check_launch("clifford_rowsum launch");
   ring_release(ticket, s);
+  return rc;
+}
+
+int qj_clifford_forms_supported(int nqubits, int m) {
+  RowsPlan p;
+  return nqubits >= 1 && nqubits <= kCliffMaxQubits && m >= 1 && rows_plan(nqubits, m + 1, &p) ? 1 : 0;
+}
+
+int qj_clifford_measurement_forms(const uint32_t* tab, int nqubits, const int32_t* qubits, int m, uint8_t* forms,
+                                  int32_t* nrandom_out, void* stream) {
+  int rc = check_tab(tab, nqubits, "clifford_measurement_forms");
+  if (rc) return rc;
+  if (m < 1 || !qubits || !forms || !nrandom_out)
+    return set_error(QJ_EVALUE, "clifford_measurement_forms: null pointer or no qubits");
+  for (int i = 0; i < m; ++i)
+    if (qubits[i] < 0 || qubits[i] >= nqubits)
+      return set_error(QJ_EVALUE, "clifford_measurement_forms: qubit %d out of range at %d", qubits[i], i);
+  RowsArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.n = nqubits;
+  a.m = m;
+  a.S = m + 1;
+  a.forms = forms;
+  a.nrandom = nrandom_out;
+  if (!launch_measure_rows<true>(const_cast<uint32_t*>(tab), a, qubits, (hipStream_t)stream, &rc))
+    return set_error(QJ_EVALUE, "clifford_measurement_forms: tableau or stream not supported");
   return rc;
 }
 
