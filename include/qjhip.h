@@ -194,6 +194,11 @@ int qj_apply_tile_pass(void* state, int dtype, int nqubits, int low_bits,
                        const int32_t* high_bits, int nhigh,
                        const qj_tile_op* ops, int nops, const void* data,
                        uint64_t data_bytes, void* stream);
+/* The same pass read from `source` (another state of the same shape, left
+ * unchanged; NULL: |0...0>) and written to `state`. */
+int qj_apply_tile_pass_from(const void* source, void* state, int dtype, int nqubits, int low_bits,
+                            const int32_t* high_bits, int nhigh, const qj_tile_op* ops, int nops, const void* data,
+                            uint64_t data_bytes, void* stream);
 
 /* Swaps of disjoint bit pairs (pairs[2j], pairs[2j+1]), j < npairs, all in one
  * read and one write of the state: the permutation of a run of SWAP gates

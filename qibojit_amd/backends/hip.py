@@ -761,16 +761,18 @@ class HipBackend(Backend):
         nqubits = circuit.nqubits
         density_matrix = bool(getattr(circuit, "density_matrix", False))
         try:
-            if initial_state is None:
+            if isinstance(initial_state, QuantumState):
+                initial_state = initial_state.state()
+            if self.fusion and (initial_state is None or self._is_plain_state(initial_state)):
+                state = self._run_fused_from(circuit.queue, initial_state, nqubits, density_matrix)
+            elif initial_state is None:
                 state = self.zero_state(nqubits, density_matrix=density_matrix)
             else:
-                if isinstance(initial_state, QuantumState):
-                    initial_state = initial_state.state()
                 dtype = _dtype_name(initial_state.dtype) if hasattr(initial_state, "dtype") else self.dtype
                 state = self.cast(initial_state, dtype=dtype, copy=True)
-            if self.fusion:
-                state = self.apply_gates_fused(circuit.queue, state, nqubits)
-            else:
+                if self.fusion:
+                    state = self.apply_gates_fused(circuit.queue, state, nqubits)
+            if not self.fusion:
                 for gate in circuit.queue:
                     if density_matrix:
                         state = gate.apply_density_matrix(self, state, nqubits)
@@ -818,9 +820,36 @@ class HipBackend(Backend):
         name = gate.__class__.__name__
         return not (name in ("M", "Align", "CallbackGate") or "Channel" in name or hasattr(gate, "coefficients"))
 
+    def _is_plain_state(self, state):
+        """A device tensor whose memory a kernel can read as the state."""
+        return (
+            isinstance(state, torch.Tensor)
+            and state.device == self._torch_device
+            and state.dtype in (torch.complex64, torch.complex128)
+            and state.is_contiguous()
+            and not state.is_conj()
+            and not state.is_neg()
+        )
+
+    def _run_fused_from(self, gates, source, nqubits, density_matrix):
+        """The state ``gates`` make of ``source`` (a plain state, left
+        unchanged, or None for |0...0>), in a new tensor.  The first tile pass
+        reads the source and writes the new state, so nothing is copied."""
+        if source is None:
+            tdt = _TORCH_DTYPES[self.dtype]
+            shape = (1 << nqubits,) * (2 if density_matrix else 1)
+        else:
+            tdt, shape = source.dtype, tuple(source.shape)
+        state = _device_empty(math.prod(shape), tdt, self._torch_device).reshape(shape)
+        return self._apply_gates_fused(gates, state, nqubits, start=(source,))
+
     def apply_gates_fused(self, gates, state, nqubits):
         """Apply ``gates`` in order with the fused tile executor."""
-        state = self._as_state(state)
+        return self._apply_gates_fused(gates, self._as_state(state), nqubits)
+
+    def _apply_gates_fused(self, gates, state, nqubits, start=None):
+        """``start`` = (source,): ``state`` is still to be filled, from
+        ``source`` or, if that is None, with |0...0>."""
         density_matrix = len(tuple(state.shape)) == 2
         shape = state.shape
         flat = state.reshape(-1)
@@ -832,8 +861,25 @@ class HipBackend(Backend):
         def launch(passes):
             # each pass is launched as soon as the planner closes it, so the
             # host converts the next pass's gates while this one runs
-            if passes:
-                tiles.run_passes(call, _ptr(flat), _NATIVE_CODES[flat.dtype], nbits, passes, npdt, self._stream())
+            nonlocal start
+            if not passes:
+                return
+            if start is not None and isinstance(passes[0], tiles.SwapPass):
+                fill()
+            from_source = start is not None
+            source = _ptr(start[0]) if from_source and start[0] is not None else None
+            start = None
+            tiles.run_passes(call, _ptr(flat), _NATIVE_CODES[flat.dtype], nbits, passes, npdt, self._stream(),
+                             source, from_source)
+
+        def fill():
+            # nothing has been written yet: the starting state itself
+            nonlocal start
+            if start[0] is None:
+                call("qj_initial_state", _ptr(flat), _NATIVE_CODES[flat.dtype], flat.numel(), self._stream())
+            else:
+                flat.copy_(start[0].reshape(-1))
+            start = None
 
         for gate in gates:
             seq = tiles.expand_fanout(gate) if gate.name == "fanout" else [gate]
@@ -855,6 +901,8 @@ class HipBackend(Backend):
                 op = tiles.gate_to_op(self._custom_matrix_c128, g, nbits) if self._is_unitary_gate(g) else None
                 if op is None or not tiles.fits_alone(op, low, max_high):
                     launch(planner.finish())
+                    if start is not None:
+                        fill()
                     st = flat.reshape(shape)
                     st = g.apply_density_matrix(self, st, nqubits) if density_matrix else g.apply(self, st, nqubits)
                     flat = self._as_state(st).reshape(-1)
@@ -863,6 +911,8 @@ class HipBackend(Backend):
                 if density_matrix:
                     launch(planner.push(tiles.column_op(op, nqubits)))
         launch(planner.finish())
+        if start is not None:
+            fill()
         return flat.reshape(shape)
 
     def assert_allclose(self, value, target, rtol=1e-7, atol=0.0):

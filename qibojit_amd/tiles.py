@@ -338,9 +338,10 @@ def encode(p, nqubits, npdtype):
     return ops, b"".join(chunks), high
 
 
-def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream):
-    """Issue one qj_apply_tile_pass (or qj_apply_bit_swaps) per pass
-    (stream-ordered, no host sync)."""
+def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream, source_ptr=None, from_source=False):
+    """Issue one tile pass (or qj_apply_bit_swaps) per pass (stream-ordered,
+    no host sync).  With ``from_source`` the first one, which must be a tile
+    pass, reads ``source_ptr`` (None: the state |0...0>) instead of the state."""
     for p in passes:
         if isinstance(p, SwapPass):
             flat = [b for pair in p.pairs for b in pair]
@@ -352,7 +353,8 @@ def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream
         harr = (ctypes.c_int32 * max(1, len(high)))(*high)
         dbuf = ctypes.create_string_buffer(data, max(1, len(data)))
         lib_call(
-            "qj_apply_tile_pass",
+            "qj_apply_tile_pass_from",
+            source_ptr if from_source else state_ptr,
             state_ptr,
             dtype_code,
             nqubits,
@@ -365,3 +367,4 @@ def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream
             len(data),
             stream,
         )
+        from_source = False
