@@ -242,6 +242,26 @@ def dominant_kernel(rows):
 
 
 # ---------------------------------------------------------------- extras --
+def planned_passes(backend, queue, n, tdtype):
+    """Passes over the state that the fused executor plans for a gate list."""
+    import ctypes
+
+    import torch
+
+    from qibojit_amd import _native
+    from qibojit_amd.records import Records
+
+    records = Records()
+    for gate in queue:
+        records.add(gate, backend._as_custom_matrix)  # pylint: disable=protected-access
+    low, max_high = backend.tile_geometry(n, tdtype)
+    code = _native.QJ_COMPLEX64 if tdtype == torch.complex64 else _native.QJ_COMPLEX128
+    passes = ctypes.c_int32(0)
+    _native.call("qj_run_gates", None, 0, None, code, n, 0, low, max_high, records.words.buffer_info()[0],
+                 len(records.words), records.params.buffer_info()[0], len(records.params), ctypes.byref(passes), None)
+    return passes.value
+
+
 def run_qft(backend, n, dtype, fused=False, reps=1):
     """QFT (H + controlled-phase ladder + final swaps) from a seeded state,
     gate by gate or through the fused tile executor.  With reps > 1 the
@@ -266,11 +286,7 @@ def run_qft(backend, n, dtype, fused=False, reps=1):
     torch.cuda.synchronize()
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     if fused:
-        from qibojit_amd import tiles
-
-        low, max_high = backend.tile_geometry(n, tdt)
-        ops = [tiles.gate_to_op(backend._as_custom_matrix, g, n) for g in c.queue]  # pylint: disable=protected-access
-        npasses = len(tiles.plan(ops, n, low, max_high))
+        npasses = planned_passes(backend, c.queue, n, tdt)
     runs = []
     for _ in range(reps):
         e0.record()

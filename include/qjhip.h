@@ -171,12 +171,15 @@ int qj_apply_block_mfma(void* state, int dtype, int nqubits,
  *     W[b] = exp(i * theta of tile bit b);
  *   QJ_TILE_SWAP: exchanges tile-local bits target[0] and target[1] (k = 2,
  *     no controls, no data), the reference's apply_swap_kernel
- *     (custom_operators/gates.py:196-216) inside the tile.
- * Dense and phase ops apply only where every bit of `local_ctrl` (tile-local
+ *     (custom_operators/gates.py:196-216) inside the tile;
+ *   QJ_TILE_SCALE: multiplies by the complex number (the state's precision)
+ *     at `data + offset`: a controlled phase, its target among the controls.
+ * Dense, phase and scale ops apply only where every bit of `local_ctrl` (tile-local
  * mask) and of `global_ctrl` (mask of out-of-tile bit positions) is 1. */
 #define QJ_TILE_DENSE 0
 #define QJ_TILE_PHASE 1
 #define QJ_TILE_SWAP 2
+#define QJ_TILE_SCALE 3
 #define QJ_TILE_MAX_K 5
 #define QJ_TILE_MAX_BITS 13
 
@@ -199,6 +202,43 @@ int qj_apply_tile_pass(void* state, int dtype, int nqubits, int low_bits,
 int qj_apply_tile_pass_from(const void* source, void* state, int dtype, int nqubits, int low_bits,
                             const int32_t* high_bits, int nhigh, const qj_tile_op* ops, int nops, const void* data,
                             uint64_t data_bytes, void* stream);
+
+/* ---- gate lists: planned into tile passes and run, one call per list ----
+ * A record is {code, ntargets, ncontrols, targets..., controls...} (qubits,
+ * qubit 0 the top bit; any number of controls except for SWAP), its
+ * parameters follow one another in `params`: the angles of RX, RY, RZ, U1 (1),
+ * U2 (2) and U3 (3), the complex128 row-major matrix on the targets (first =
+ * MSB, at most QJ_TILE_MAX_K) of DENSE and DENSE_BITS, nothing otherwise.
+ * With density != 0 the state is the 2^nqubits x 2^nqubits matrix rho and a
+ * gate U maps it to U rho U^+; DENSE_BITS acts once, on the listed qubits of
+ * the 2 nqubits (row qubit q = q, column qubit q = nqubits + q).
+ * from_source != 0: `state` is filled from `source` (NULL: |0...0>) on the way.
+ * low_bits, max_high: the tile's low run and most further bits.
+ * *npasses (host, may be NULL) gets the number of passes; state == NULL only
+ * plans.  Stream-ordered; the records may be reused on return. */
+#define QJ_GATE_DENSE 0
+#define QJ_GATE_DENSE_BITS 1
+#define QJ_GATE_SWAP 2
+#define QJ_GATE_X 3
+#define QJ_GATE_Y 4
+#define QJ_GATE_Z 5
+#define QJ_GATE_H 6
+#define QJ_GATE_S 7
+#define QJ_GATE_SDG 8
+#define QJ_GATE_T 9
+#define QJ_GATE_TDG 10
+#define QJ_GATE_SX 11
+#define QJ_GATE_SXDG 12
+#define QJ_GATE_RX 13
+#define QJ_GATE_RY 14
+#define QJ_GATE_RZ 15
+#define QJ_GATE_U1 16
+#define QJ_GATE_U2 17
+#define QJ_GATE_U3 18
+#define QJ_GATE_LAST 18
+int qj_run_gates(const void* source, int from_source, void* state, int dtype, int nqubits, int density, int low_bits,
+                 int max_high, const int32_t* recs, int64_t nwords, const double* params, int64_t nparams,
+                 int32_t* npasses, void* stream);
 
 /* Swaps of disjoint bit pairs (pairs[2j], pairs[2j+1]), j < npairs, all in one
  * read and one write of the state: the permutation of a run of SWAP gates

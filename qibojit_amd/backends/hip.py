@@ -38,6 +38,7 @@ from qibojit_amd import tiles
 from qibojit_amd._qibo import gates as gate_classes
 from qibojit_amd.backends.matrices import KernelMatrices
 from qibojit_amd.fusion import GATE_OPS, channel_superoperator, fused_matrix
+from qibojit_amd.records import DENSE_BITS, GATE_CODES, Records
 
 
 _TORCH_DTYPES = {
@@ -61,6 +62,12 @@ _REAL_OF = {torch.complex64: torch.float32, torch.complex128: torch.float64}
 # apply_density_matrix of the channels that are plain operator sums; a class
 # with its own (qibo's depolarizing and thermal relaxation channels) keeps it
 _CHANNEL_APPLY = getattr(getattr(gate_classes, "Channel", None), "apply_density_matrix", None)
+
+
+# Gates planned together by the fused executor.  The planner looks through all
+# of them for what a pass can take; the device waits for the first run's
+# records, about 2 us each.
+_RECORDS_PER_RUN = 512
 
 
 def _dtype_name(dtype):
@@ -855,34 +862,27 @@ class HipBackend(Backend):
         flat = state.reshape(-1)
         nbits = 2 * nqubits if density_matrix else nqubits
         low, max_high = self.tile_geometry(nbits, flat.dtype)
-        npdt = np.complex64 if flat.dtype == torch.complex64 else np.complex128
-        planner = tiles.Planner(nbits, low, max_high)
+        code = _NATIVE_CODES[flat.dtype]
+        records = Records()
 
-        def launch(passes):
-            # each pass is launched as soon as the planner closes it, so the
-            # host converts the next pass's gates while this one runs
+        def flush():
             nonlocal start
-            if not passes:
+            if records.count == 0 and start is None:
                 return
-            if start is not None and isinstance(passes[0], tiles.SwapPass):
-                fill()
-            from_source = start is not None
-            source = _ptr(start[0]) if from_source and start[0] is not None else None
+            source = _ptr(start[0]) if start is not None and start[0] is not None else None
+            call("qj_run_gates", source, int(start is not None), _ptr(flat), code, nqubits, int(density_matrix), low,
+                 max_high, records.words.buffer_info()[0], len(records.words), records.params.buffer_info()[0],
+                 len(records.params), None, self._stream())
             start = None
-            tiles.run_passes(call, _ptr(flat), _NATIVE_CODES[flat.dtype], nbits, passes, npdt, self._stream(),
-                             source, from_source)
-
-        def fill():
-            # nothing has been written yet: the starting state itself
-            nonlocal start
-            if start[0] is None:
-                call("qj_initial_state", _ptr(flat), _NATIVE_CODES[flat.dtype], flat.numel(), self._stream())
-            else:
-                flat.copy_(start[0].reshape(-1))
-            start = None
+            records.clear()
 
         for gate in gates:
-            seq = tiles.expand_fanout(gate) if gate.name == "fanout" else [gate]
+            if type(gate).__name__ in GATE_CODES:  # named gates, the common case
+                records.add(gate, self._custom_matrix_c128)
+                if records.count >= _RECORDS_PER_RUN:
+                    flush()
+                continue
+            seq = tiles.expand_fanout(gate) if gate.name == "fanout" else (gate,)
             for g in seq:
                 if density_matrix and type(g).apply_density_matrix is _CHANNEL_APPLY:
                     # a channel on one or two qubits: its superoperator is a
@@ -891,28 +891,19 @@ class HipBackend(Backend):
                     # passes of their own otherwise; 39.6 -> 1.9 ms for the circuit)
                     block, matrix = self._channel_superoperator(g)
                     if block is not None:
-                        targets = [nbits - 1 - q for q in block] + [nqubits - 1 - q for q in block]
-                        op = tiles.DenseOp(targets, (), matrix)
-                        if tiles.fits_alone(op, low, max_high):
-                            launch(planner.push(op))
-                            continue
-                # ops are built from complex128 matrices (exact phase angles)
-                # and cast to the state's precision when a pass is encoded
-                op = tiles.gate_to_op(self._custom_matrix_c128, g, nbits) if self._is_unitary_gate(g) else None
-                if op is None or not tiles.fits_alone(op, low, max_high):
-                    launch(planner.finish())
-                    if start is not None:
-                        fill()
-                    st = flat.reshape(shape)
-                    st = g.apply_density_matrix(self, st, nqubits) if density_matrix else g.apply(self, st, nqubits)
-                    flat = self._as_state(st).reshape(-1)
+                        records.add_dense(DENSE_BITS, block + [q + nqubits for q in block], (), matrix)
+                        continue
+                # matrices are complex128 (exact phase angles), cast to the
+                # state's precision when a pass is encoded
+                if self._is_unitary_gate(g) and records.add(g, self._custom_matrix_c128):
+                    if records.count >= _RECORDS_PER_RUN:
+                        flush()
                     continue
-                launch(planner.push(op))
-                if density_matrix:
-                    launch(planner.push(tiles.column_op(op, nqubits)))
-        launch(planner.finish())
-        if start is not None:
-            fill()
+                flush()
+                st = flat.reshape(shape)
+                st = g.apply_density_matrix(self, st, nqubits) if density_matrix else g.apply(self, st, nqubits)
+                flat = self._as_state(st).reshape(-1)
+        flush()
         return flat.reshape(shape)
 
     def assert_allclose(self, value, target, rtol=1e-7, atol=0.0):

@@ -16,7 +16,7 @@ LIB = os.path.join(HERE, "libqjhip.so")
 ARCH = os.environ.get("QJ_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["qj_runtime.hip", "qj_gates.hip", "qj_ops.hip", "qj_tile.hip", "qj_group.hip", "qj_mfma.hip",
+SOURCES = ["qj_runtime.hip", "qj_gates.hip", "qj_ops.hip", "qj_tile.hip", "qj_circuit.hip", "qj_group.hip", "qj_mfma.hip",
            "qj_clifford.hip"]
 
 CFLAGS = [

@@ -483,6 +483,8 @@ __global__ void __launch_bounds__(BSMAX, WPE)
         const cplx<R>* d = reinterpret_cast<const cplx<R>*>(ldata + uni((int)op.loff));
         if (kind == kRegPhase)
           reg_phase<R, NRB>(x, f[uni(op.fidx)], d, NT, tid, rcm);
+        else if (kind == kRegScale)
+          reg_scale<R, NRB>(x, *d, rcm);
         else
           reg_dense_any<R, NRB>(x, kind, uni(op.mask), d, rcm);
       }
@@ -613,9 +615,18 @@ static void lds_kernel_data(const qj_tile_op* ops, int nops, const char* data, i
     const qj_tile_op& op = ops[o];
     if (op.kind == QJ_TILE_DENSE) {
       ops_out[o].offset = put(data + op.offset, ((size_t)1 << (2 * op.k)) * sizeof(cplx<R>));
-    } else if (op.kind == QJ_TILE_PHASE) {
+    } else if (op.kind == QJ_TILE_PHASE || op.kind == QJ_TILE_SCALE) {
       const cplx<R>* src = reinterpret_cast<const cplx<R>*>(data + op.offset + 16);
       const size_t na = size_t(1) << ga, nb = size_t(1) << gb;
+      std::vector<cplx<R>> flat;
+      if (op.kind == QJ_TILE_SCALE) {  // a phase with its factor in every entry of OA
+        cplx<R> z;
+        std::memcpy(&z, data + op.offset, sizeof(z));
+        flat.assign(na + nb + (size_t)TB, mk<R>(1, 0));
+        std::fill(flat.begin(), flat.begin() + (long)na, z);
+        src = flat.data();
+        ops_out[o].kind = QJ_TILE_PHASE;
+      }
       const cplx<R>* w = src + na + nb;
       std::vector<cplx<R>> blk(na + nb + (size_t(1) << la) + (size_t(1) << (TB - la)));
       std::memcpy(blk.data(), src, (na + nb) * sizeof(cplx<R>));
@@ -774,6 +785,10 @@ static int tile_pass_impl(const void* source, void* state, int nqubits, int L, c
                          o, hh[0], hh[1], hh[2], ga, gb, TB);
       const u64 need = op.offset + 16 + ((u64(1) << ga) + (u64(1) << gb) + (u64)TB) * sizeof(cplx<R>);
       if (need > data_bytes) return set_error(QJ_EVALUE, "apply_tile_pass: op %d phase tables outside data", o);
+    } else if (op.kind == QJ_TILE_SCALE) {
+      if (op.offset % 16) return set_error(QJ_EVALUE, "apply_tile_pass: op %d data offset not 16-aligned", o);
+      if (op.offset + sizeof(cplx<R>) > data_bytes)
+        return set_error(QJ_EVALUE, "apply_tile_pass: op %d factor outside data", o);
     } else {
       return set_error(QJ_EVALUE, "apply_tile_pass: op %d has unknown kind %d", o, op.kind);
     }

@@ -66,6 +66,7 @@ constexpr int kRegDense = 0;      // complex matrix
 constexpr int kRegPhase = 1;
 constexpr int kRegDenseReal = 2;  // 2x2 matrix with zero imaginary parts
 constexpr int kRegHad = 3;        // h * [[1, 1], [1, -1]], no controls: factor h deferred
+constexpr int kRegScale = 4;      // one factor where every control holds
 // Deferred factors per plan: the unscaled butterflies grow amplitudes by
 // at most sqrt(2) each, 2^16 for 32 of them, far from overflow in FP32.
 constexpr int kRegMaxHad = 32;
@@ -349,6 +350,21 @@ __host__ __device__ __forceinline__ void reg_phase(cplx<R> (&x)[1 << NRB], cplx<
   }
 }
 
+// Scale op: the registers whose bits satisfy the controls times z.  One
+// product per such amplitude (a phase op takes two and its tables).  The
+// controls stay a runtime mask (uniform branches): compile-time cases merge
+// into indexed stores and move the tile to scratch.
+template <typename R, int NRB>
+__host__ __device__ __forceinline__ void reg_scale(cplx<R> (&x)[1 << NRB], cplx<R> z, int rcm) {
+#pragma unroll
+  for (int r = 0; r < (1 << NRB); ++r) {
+    if ((r & rcm) != rcm) continue;
+    const R t_re = x[r].im * z.im, t_im = x[r].re * z.im;
+    x[r].re = qfma(x[r].re, z.re, -t_re);
+    x[r].im = qfma(x[r].im, z.re, t_im);
+  }
+}
+
 // Out-of-tile factor of a phase op for tile t (tables at `tab`).
 template <typename R>
 __host__ __device__ __forceinline__ cplx<R> reg_phase_outside(const cplx<R>* __restrict__ tab, int ga, u64 t) {
@@ -524,7 +540,7 @@ inline bool reg_plan(const RegPlanIn& in, std::vector<char>& blob) {
       const qj_tile_op& op = in.ops[p.op];
       RegOp& ro = rops[i];
       std::memset(&ro, 0, sizeof(ro));
-      ro.kind = op.kind == QJ_TILE_PHASE ? kRegPhase : kRegDense;
+      ro.kind = op.kind == QJ_TILE_PHASE ? kRegPhase : op.kind == QJ_TILE_SCALE ? kRegScale : kRegDense;
       ro.gctrl = op.global_ctrl;
       ro.fidx = -1;
       // local controls: thread-bit part (tile bits) and register-index part
@@ -578,6 +594,8 @@ inline bool reg_plan(const RegPlanIn& in, std::vector<char>& blob) {
           }
         }
         ro.loff = put(ldata, mat.data(), mat.size());
+      } else if (op.kind == QJ_TILE_SCALE) {
+        ro.loff = put(ldata, in.data + op.offset, (size_t)in.esize);
       } else {
         // ABI block: int32 {ga, gb, tb, pad}, OA[2^ga], OB[2^gb], W[tb] (logical bits)
         const char* src = in.data + op.offset + 16;

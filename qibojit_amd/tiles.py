@@ -1,4 +1,9 @@
-"""Planner of fused tile passes (the gate-fusion executor).
+"""Tile passes in Python: ops, the in-order planner and the encoding of
+``qj_apply_tile_pass``.
+
+The fused executor plans in the library (``qj_run_gates``, which also moves
+gates past others they commute with); this module states the pass format op
+by op, for callers of the pass entry points and for checking them.
 
 A circuit segment of unitary gates is cut into passes.  Each pass streams
 the state once through LDS tiles (``qj_apply_tile_pass``) whose bits are
@@ -338,10 +343,9 @@ def encode(p, nqubits, npdtype):
     return ops, b"".join(chunks), high
 
 
-def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream, source_ptr=None, from_source=False):
-    """Issue one tile pass (or qj_apply_bit_swaps) per pass (stream-ordered,
-    no host sync).  With ``from_source`` the first one, which must be a tile
-    pass, reads ``source_ptr`` (None: the state |0...0>) instead of the state."""
+def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream):
+    """Issue one qj_apply_tile_pass (or qj_apply_bit_swaps) per pass
+    (stream-ordered, no host sync)."""
     for p in passes:
         if isinstance(p, SwapPass):
             flat = [b for pair in p.pairs for b in pair]
@@ -353,8 +357,7 @@ def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream
         harr = (ctypes.c_int32 * max(1, len(high)))(*high)
         dbuf = ctypes.create_string_buffer(data, max(1, len(data)))
         lib_call(
-            "qj_apply_tile_pass_from",
-            source_ptr if from_source else state_ptr,
+            "qj_apply_tile_pass",
             state_ptr,
             dtype_code,
             nqubits,
@@ -367,4 +370,3 @@ def run_passes(lib_call, state_ptr, dtype_code, nqubits, passes, npdtype, stream
             len(data),
             stream,
         )
-        from_source = False
