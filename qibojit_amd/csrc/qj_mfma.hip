@@ -38,6 +38,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kMfmaBlock = 256;  // 4 waves, 32 columns each per step
 constexpr u64 kMfmaMaxGrid = 8192;
+constexpr u64 kMfmaMinGrid = 512;  // two workgroups per CU
 
 // Workgroups of the 3M kernel: complex64 K = 4 131072 and K = 5 32768,
 // complex128 K = 4 524288 and K = 5 8192 (the complex128 5-target kernel,
@@ -211,18 +212,20 @@ __global__ void __launch_bounds__(kMfmaBlock)
   const int q = lane >> 4, n = lane & 15;
   // the three real NR x NR blocks are read from global memory once per
   // workgroup (not once per wave), then each wave takes its A operands
-  __shared__ R umat[3 * NR * NR];
-  for (int i = threadIdx.x; i < 3 * NR * NR; i += kMfmaBlock) umat[i] = u3[i];
+  // (rows padded by one entry: the 16 rows a K-step reads start on 16 banks)
+  constexpr int US = NR + 1;
+  __shared__ R umat[3 * NR * US];
+  for (int i = threadIdx.x; i < 3 * NR * NR; i += kMfmaBlock) umat[(i / NR) * US + i % NR] = u3[i];
   __syncthreads();
   R ur[T][S], ui[T][S], us[T][S];
 #pragma unroll
   for (int t = 0; t < T; ++t)
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      const int e = (16 * t + n) * NR + 4 * s + q;
+      const int e = (16 * t + n) * US + 4 * s + q;
       ur[t][s] = umat[e];
-      ui[t][s] = umat[NR * NR + e];
-      us[t][s] = umat[2 * NR * NR + e];
+      ui[t][s] = umat[NR * US + e];
+      us[t][s] = umat[2 * NR * US + e];
     }
   // chunk-local index of this lane's column (targets inserted as zeros)
   const unsigned colbase = STAGE ? (unsigned)(insert_bits((u64)n, ins) & lowmask) : 0u;
@@ -422,11 +425,17 @@ static int block_impl(void* state, int nqubits, const int32_t* target_bits, int 
   // 32 qubits complex64 and 30 qubits complex128 over caps of 8192..2^21
   const u64 cap = mfma_grid_cap(sizeof(R) == 8, K);
   if (grid > cap) grid = cap;
-  // at least two 16-column groups per wave: one group per wave reloads the
-  // matrix for every 2^K x 16 amplitudes (complex128 K = 4 with a control:
-  // 58% of the HBM peak at one group per wave, 68% at two or more)
-  const u64 two_per_wave = ncols / (2 * 16 * (kMfmaBlock / 64));
-  if (two_per_wave >= 1 && grid > two_per_wave) grid = two_per_wave;
+  // 16-column groups per wave, so that a workgroup's matrix load is spread over
+  // them: two for K = 4 (complex128 with a control: 58% of the HBM peak at one,
+  // 68% at two or more); eight for K = 5, whose matrix is four times larger,
+  // fewer (at least two) where that leaves under two workgroups per CU.
+  // K = 5, 27 qubits complex64: 502 us at two, 441 at four, 426 at eight, 424
+  // at 16 (683 before the rows were padded); 24 qubits 71 / 67 / 60 / 63,
+  // complex128 131 / 117 / 110 / 107; 22 qubits 30 / 31 / 33 / 43.
+  u64 per_wave = K == 5 ? 8 : 2;
+  while (per_wave > 2 && ncols / (per_wave * 16 * (kMfmaBlock / 64)) < kMfmaMinGrid) per_wave /= 2;
+  const u64 spread = ncols / (per_wave * 16 * (kMfmaBlock / 64));
+  if (spread >= 1 && grid > spread) grid = spread;
   // The lowest K + 4 bits hold exactly the targets and 4 column bits: a
   // wave's 16 columns are one contiguous run (staged through LDS).
   const int low = K + 4;
