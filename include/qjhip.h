@@ -323,6 +323,15 @@ int qj_tfim_batch(const void* psi, void* out, int dtype, int nqubits,
 int qj_ansatz_lds(int dtype, const int32_t* desc, int ncirc, const void* mats,
                   uint64_t mats_len, double g, double* energies, int nqmax,
                   int nblocks, void* stream);
+/* The 2x2 matrices of ansatz circuits (per layer RY then RZ on every qubit)
+ * from their angles.  Circuit c has the record {parameter offset, slot offset,
+ * n, layers, slots per layer, map offset} (device int64 x 6); its angles are
+ * those of the ansatz (layer l: n of RY, then n of RZ, qubit order).  Bit p
+ * (qubit n-1-p) of layer l goes to slot `slot offset + l * slots per layer +
+ * map[map offset + p]` of `mats` (nslots slots of steps x 4 numbers): RZ RY for
+ * steps = 1, RY and RZ one after the other for steps = 2. */
+int qj_ansatz_mats(const double* params, uint64_t nparams, const int64_t* recs, int nrecs, const int32_t* map,
+                   uint64_t nmap, void* mats, int dtype, uint64_t nslots, int steps, void* stream);
 /* out[r] = sum_{c < ncols} in[r * ncols + c] in FP64, fixed order. */
 int qj_reduce_rows(const double* in, uint64_t nrows, uint64_t ncols,
                    double* out, void* stream);

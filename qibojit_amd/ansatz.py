@@ -170,6 +170,13 @@ def _tfim_cols(dim, tdtype):
     return _cols(dim // (4 if tdtype == torch.complex64 else 2), MAX_COLS)
 
 
+def pass_slots(passes, rows, width):
+    """Matrix slot of every bit in a layer of [pass, row, place] slots, for row
+    0 (row r adds r * width)."""
+    slots = {bit: (i * rows) * width + a for i, ps in enumerate(passes) for a, bit in enumerate(ps.bits) if bit in ps.rot}
+    return [slots[bit] for bit in range(len(slots))]
+
+
 class AnsatzEngine:
     """Batched energies and adjoint gradients of one ansatz shape.
 
@@ -224,6 +231,7 @@ class AnsatzEngine:
                       for ps in self.passes_a]
         self.tfim_partials = torch.zeros((self.batch, self.tfim_cols), dtype=torch.float64, device=self.device)
         self.energies_dev = torch.zeros(self.batch, dtype=torch.float64, device=self.device)
+        self._mats = {}
 
     # kept for callers that inspect the register grouping
     @property
@@ -247,6 +255,24 @@ class AnsatzEngine:
     def _qubit_of(self, bit):
         return self.ansatz.nqubits - 1 - bit
 
+    def _device_mats(self, p, passes, width, steps):
+        """The matrices of ``_forward_mats`` (steps 1) or ``_adjoint_mats``
+        (steps 2), built by a kernel from the angles."""
+        n, nl, b = self.ansatz.nqubits, self.ansatz.nlayers, self.batch
+        with torch.cuda.stream(self.stream):
+            if steps not in self._mats:
+                recs = [(r * self.ansatz.nparams, r * width, n, nl, len(passes) * b * width, 0) for r in range(b)]
+                self._mats[steps] = (
+                    torch.tensor(recs, dtype=torch.int64, device=self.device),
+                    torch.tensor(pass_slots(passes, b, width), dtype=torch.int32, device=self.device),
+                    torch.zeros((nl, len(passes), b, width, steps, 4), dtype=self.tdtype, device=self.device),
+                )
+            angles = torch.tensor(np.ascontiguousarray(p), device=self.device)
+            recs, slots, mats = self._mats[steps]
+            call("qj_ansatz_mats", _vp(angles), angles.numel(), _vp(recs), b, _vp(slots), n, _vp(mats), self.code,
+                 mats.numel() // (4 * steps), steps, self._stream())
+        return mats
+
     def _params(self, params):
         p = params.detach().cpu().numpy() if isinstance(params, torch.Tensor) else np.asarray(params)
         p = np.asarray(p, dtype=np.float64)
@@ -254,6 +280,7 @@ class AnsatzEngine:
             raise ValueError(f"Expected parameters of shape {(self.batch, self.ansatz.nparams)}, got {p.shape}.")
         return p
 
+    # the layouts of _device_mats, on the host
     def _forward_mats(self, p):
         """[L, P, B, W, 1, 4]: RZ @ RY per rotated bit at its place in the pass."""
         ang = self.ansatz.angles(p)  # (B, L, 2, n)
@@ -302,7 +329,7 @@ class AnsatzEngine:
         """Evolve |0...0> through the ansatz for every parameter set; the
         states are left before the last ladder (``self.psi[self.cur]``)."""
         p = self._params(params)
-        mats = self._forward_mats(p)
+        mats = self._device_mats(p, self.passes_f, self.width_f, 1)
         psi = self.psi
         cur = 0
         for layer in range(self.ansatz.nlayers):
@@ -318,7 +345,6 @@ class AnsatzEngine:
                                self.width_f * 4, None, self.cols_f[i])
         self.cur = cur
         self._forward_key = p.tobytes()
-        self._mats_keepalive = mats
         return p
 
     def energies(self, params):
@@ -350,7 +376,7 @@ class AnsatzEngine:
             self.run_forward(p)
         if self.lam is None:
             self.lam = torch.empty_like(self.psi)
-        mats = self._adjoint_mats(p)
+        mats = self._device_mats(p, self.passes_a, self.width_a, 2)
         nl, npass, width = self.ansatz.nlayers, len(self.passes_a), self.width_a
         ncols = self.cols_a
         partials = torch.zeros((nl, npass, width * 2, self.batch, ncols), dtype=torch.float64, device=self.device)

@@ -39,6 +39,7 @@ from qibojit_amd.ansatz import (
     ROT_BLOCK,
     TILE_BITS,
     HardwareEfficientAnsatz,
+    pass_slots,
     register_passes,
     ry_matrices,
     rz_matrices,
@@ -46,7 +47,6 @@ from qibojit_amd.ansatz import (
 )
 
 _CODES = {torch.complex64: _native.QJ_COMPLEX64, torch.complex128: _native.QJ_COMPLEX128}
-_NP = {torch.complex64: np.complex64, torch.complex128: np.complex128}
 LDS_MAX_QUBITS = {torch.complex64: 13, torch.complex128: 12}
 LDS_MIN_QUBITS = 2
 
@@ -62,23 +62,27 @@ def _fused_layers(n, nlayers, params):
     return m[:, ::-1].reshape(nlayers, n, 4)
 
 
+def _passes(n, k):
+    return tile_passes(n) if k is None else register_passes(n, k)
+
+
 class _PassGroup:
     """Device buffers and launch list of the pass path for one qubit count:
     register passes of k bits, or (k = None) LDS tile passes."""
 
-    def __init__(self, n, members, layers, k, tdtype, device, tfim_cols=64):
+    def __init__(self, n, members, layers, k, mats, device, tfim_cols=64):
         self.n, self.members, self.k = n, members, k
         self.layers = np.asarray(layers)
         cnt = len(members)
         self.cnt = cnt
         self.dim = 1 << n
         self.lmax = int(self.layers.max())
-        self.passes = tile_passes(n) if k is None else register_passes(n, k)
+        self.passes = _passes(n, k)
         self.width = max(len(ps.bits) for ps in self.passes)
         self.bits = [i32_array(ps.bits) for ps in self.passes]
         self.rotmask = [sum(1 << a for a, b in enumerate(ps.bits) if b in ps.rot) for ps in self.passes]
-        self.psi = torch.empty((2, cnt, self.dim), dtype=tdtype, device=device)
-        self.mats = torch.zeros((self.lmax, len(self.passes), cnt, self.width, 1, 4), dtype=tdtype, device=device)
+        self.psi = torch.empty((2, cnt, self.dim), dtype=mats.dtype, device=device)
+        self.mats = mats.view(self.lmax, len(self.passes), cnt, self.width, 1, 4)
         self.sel = []
         for layer in range(self.lmax):
             active = np.nonzero(self.layers > layer)[0]
@@ -91,16 +95,6 @@ class _PassGroup:
         self.partials = torch.zeros((cnt, self.tfim_cols), dtype=torch.float64, device=device)
         self.cols = [int(min(self.dim >> TILE_BITS, 65535)) if ps.kind == "tile"
                      else int(min(-(-(self.dim >> len(ps.bits)) // ROT_BLOCK), 65535)) for ps in self.passes]
-
-    def pack(self, fused):
-        """fused: list over members of (L_c, n, 4) -> device matrices."""
-        host = np.zeros(tuple(self.mats.shape), dtype=_NP[self.mats.dtype])
-        for s, m in enumerate(fused):
-            for i, ps in enumerate(self.passes):
-                for a, bit in enumerate(ps.bits):
-                    if bit in ps.rot:
-                        host[: m.shape[0], i, s, a, 0] = m[:, bit]
-        self.mats.copy_(torch.from_numpy(host))
 
     def launch(self, code, g, stream, energies_out):
         psi = self.psi
@@ -166,21 +160,49 @@ class AnsatzBatch:
             lds_circ = self.order[: self.nlds]
             sizes = [self.shapes[c][1] * self.shapes[c][0] * 4 for c in lds_circ]
             offs = np.concatenate([[0], np.cumsum(sizes)[:-1]]).astype(np.int64)
-            self.lds_offsets = offs
-            self.lds_mats = torch.zeros(int(sum(sizes)), dtype=self.tdtype, device=self.device)
             desc = np.zeros((self.nlds, 4), dtype=np.int64)
             for j, c in enumerate(lds_circ):
                 desc[j] = (self.shapes[c][0], self.shapes[c][1], offs[j] & 0xFFFFFFFF, offs[j] >> 32)
             self.lds_desc = torch.from_numpy(desc.astype(np.uint32).view(np.int32)).to(self.device)
             self.lds_nqmax = int(max(self.shapes[c][0] for c in lds_circ))
             self.lds_blocks = int(lds_blocks or min(self.nlds, 1024))
+        # every matrix of the batch in one buffer of 2x2 slots: the LDS path's
+        # circuits, then one part per pass group; a record per circuit says
+        # where qj_ansatz_mats finds its angles and puts its matrices
+        poffs = np.concatenate([[0], np.cumsum([2 * n * nl for n, nl in self.shapes])]).astype(np.int64)
+        recs, slots, at = [], [], 0
+        if self.nlds:
+            first = {}
+            for c in self.order[: self.nlds]:
+                n, nl = self.shapes[c]
+                if n not in first:
+                    first[n] = len(slots)
+                    slots += range(n)
+                recs.append((poffs[c], at, n, nl, n, first[n]))
+                at += n * nl
         # pass path, one group per qubit count
-        self.pass_groups = []
-        pos = self.nlds
+        groups = []
         for n in sorted({int(v) for v in sorted_n[self.nlds:]}):
             members = [c for c in self.order[self.nlds:] if self.shapes[c][0] == n]
+            layers = [self.shapes[c][1] for c in members]
             k = None if self.plan[n][0] == "tile" else self.plan[n][1]
-            grp = _PassGroup(n, members, [self.shapes[c][1] for c in members], k, self.tdtype, self.device)
+            passes = _passes(n, k)
+            width = max(len(ps.bits) for ps in passes)
+            per_layer = len(passes) * len(members) * width
+            groups.append((n, members, layers, k, at, per_layer * max(layers)))
+            recs += [(poffs[c], at + s * width, n, nl, per_layer, len(slots))
+                     for s, (c, nl) in enumerate(zip(members, layers))]
+            slots += pass_slots(passes, len(members), width)
+            at += per_layer * max(layers)
+        self.nparams = int(poffs[-1])
+        self.mats = torch.zeros((at, 4), dtype=self.tdtype, device=self.device)
+        self.mat_recs = torch.tensor(np.array(recs, dtype=np.int64), device=self.device)
+        self.mat_slots = torch.tensor(slots, dtype=torch.int32, device=self.device)
+        self.lds_mats = self.mats[: sum(self.shapes[c][0] * self.shapes[c][1] for c in self.order[: self.nlds])]
+        self.pass_groups = []
+        pos = self.nlds
+        for n, members, layers, k, first_slot, count in groups:
+            grp = _PassGroup(n, members, layers, k, self.mats[first_slot: first_slot + count], self.device)
             grp.offset = pos
             pos += len(members)
             self.pass_groups.append(grp)
@@ -191,17 +213,18 @@ class AnsatzBatch:
         """params[c]: the 2 * n * L angles of circuit c (original order)."""
         if len(params) != len(self.shapes):
             raise ValueError("One parameter vector per circuit is required.")
-        fused = []
+        angles = []
         for c, (n, nl) in enumerate(self.shapes):
             p = np.asarray(params[c], dtype=np.float64)
             if p.size != 2 * n * nl:
                 raise ValueError(f"Circuit {c} needs {2 * n * nl} parameters, got {p.size}.")
-            fused.append(_fused_layers(n, nl, p))
-        if self.nlds:
-            host = np.concatenate([fused[c].reshape(-1) for c in self.order[: self.nlds]]).astype(_NP[self.tdtype])
-            self.lds_mats.copy_(torch.from_numpy(host))
-        for grp in self.pass_groups:
-            grp.pack([fused[c] for c in grp.members])
+            angles.append(p.reshape(-1))
+        if not angles:
+            return
+        dev = torch.tensor(np.concatenate(angles), device=self.device)
+        call("qj_ansatz_mats", _vp(dev), self.nparams, _vp(self.mat_recs), len(self.shapes), _vp(self.mat_slots),
+             self.mat_slots.numel(), _vp(self.mats), self.code, self.mats.shape[0], 1, self._stream())
+        torch.cuda.current_stream(self.device).synchronize()  # the run may be enqueued on another stream
 
     # --------------------------------------------------------- execution --
     def _stream(self):
