@@ -332,6 +332,17 @@ int qj_ansatz_lds(int dtype, const int32_t* desc, int ncirc, const void* mats,
  * steps = 1, RY and RZ one after the other for steps = 2. */
 int qj_ansatz_mats(const double* params, uint64_t nparams, const int64_t* recs, int nrecs, const int32_t* map,
                    uint64_t nmap, void* mats, int dtype, uint64_t nslots, int steps, void* stream);
+/* One step of several groups of states in one launch.  Entry k (host int64,
+ * QJ_STEP_WORDS words) is {n, count, src, dst, ladder, mats, mats per state, ka,
+ * kb, bits[10]}: `count` states of n >= 12 qubits, 2^n numbers apart, from
+ * states + src (src = -1: |0...0>) to states + dst (even offsets; src == dst in
+ * place, otherwise disjoint, always so with `ladder`).  `ladder` applies the
+ * CNOT ladder (out[k] = in[k ^ (k >> 1)]) first; then the ka + kb bits (ka 1..5,
+ * kb 0..5) are rotated in their order by the 2x2 matrices from slot `mats`
+ * (plus the state's index times `mats per state`) of 4 numbers each. */
+#define QJ_STEP_WORDS 19
+int qj_ansatz_step(void* states, int dtype, uint64_t states_len, const void* mats, uint64_t mats_len,
+                   const int64_t* entries, int nentries, void* stream);
 /* out[r] = sum_{c < ncols} in[r * ncols + c] in FP64, fixed order. */
 int qj_reduce_rows(const double* in, uint64_t nrows, uint64_t ncols,
                    double* out, void* stream);

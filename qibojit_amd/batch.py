@@ -8,10 +8,12 @@ paths, chosen per n by :func:`autotune` (or given as a plan):
   a persistent kernel, runs whole circuits inside one workgroup's LDS and
   writes only their energies; one launch serves every LDS-path circuit.
 * ``("pass", k)``: the states of all circuits with this n sit back to back
-  in two ping-pong buffers and every layer is ceil(n/k) launches of
-  ``qj_rot_pass`` over the circuits still running at that layer (the ladder
-  is folded into the next layer's first pass), then one ``qj_tfim_batch``
-  and ``qj_reduce_rows`` give the FP64 energies.
+  in two ping-pong buffers.  Every layer rotates the bits in the order of its
+  ceil(n/k) register groups: at n >= 12 in steps of up to 10 bits, one
+  ``qj_ansatz_step`` launch for the steps of all qubit counts, below that one
+  ``qj_rot_pass`` per group, always over the circuits still running at that
+  layer (the ladder is folded into the next layer's first pass).  Then one
+  ``qj_tfim_batch`` and ``qj_reduce_rows`` give the FP64 energies.
 * ``("tile",)``: as ``pass`` with LDS tile passes (``qj_rot_tile_pass``,
   12 bits each, complex64, n >= 12).
 
@@ -39,6 +41,7 @@ from qibojit_amd.ansatz import (
     ROT_BLOCK,
     TILE_BITS,
     HardwareEfficientAnsatz,
+    PassSpec,
     pass_slots,
     register_passes,
     ry_matrices,
@@ -62,31 +65,53 @@ def _fused_layers(n, nlayers, params):
     return m[:, ::-1].reshape(nlayers, n, 4)
 
 
-def _passes(n, k):
-    return tile_passes(n) if k is None else register_passes(n, k)
+STEP_BITS, STEP_TILE, STEP_WORDS = 10, 12, 19
+
+
+def step_passes(nbits, k, run):
+    """The rotation order of ``register_passes(nbits, k)`` in steps of up to
+    ``STEP_BITS`` bits whose tile (those bits and the lowest others, 12 bits)
+    holds bits 0..run-1, so that its loads are whole 128-byte lines."""
+    order = [b for ps in register_passes(nbits, k) for b in ps.bits]
+    passes = []
+    while order:
+        for count in range(min(STEP_BITS, len(order)), 0, -1):
+            bits = order[:count]
+            others = [b for b in range(nbits) if b not in bits]
+            if set(range(run)) <= set(bits + others[: STEP_TILE - count]):
+                break
+        passes.append(PassSpec("step", bits, bits))
+        order = order[count:]
+    return passes
+
+
+def _passes(n, k, tdtype):
+    if k is None:
+        return tile_passes(n)
+    if n < STEP_TILE:
+        return register_passes(n, k)
+    return step_passes(n, k, 4 if tdtype == torch.complex64 else 3)
 
 
 class _PassGroup:
     """Device buffers and launch list of the pass path for one qubit count:
-    register passes of k bits, or (k = None) LDS tile passes."""
+    register passes of k bits (in steps, at n >= 12), or (k = None) LDS tile
+    passes.  ``psi``: its part of the batch's states; members in descending
+    order of layers, so that the first ones are still running."""
 
-    def __init__(self, n, members, layers, k, mats, device, tfim_cols=64):
-        self.n, self.members, self.k = n, members, k
+    def __init__(self, n, members, layers, passes, psi, mats, device, tfim_cols=64):
+        self.n, self.members = n, members
         self.layers = np.asarray(layers)
         cnt = len(members)
         self.cnt = cnt
         self.dim = 1 << n
         self.lmax = int(self.layers.max())
-        self.passes = _passes(n, k)
+        self.passes = passes
         self.width = max(len(ps.bits) for ps in self.passes)
         self.bits = [i32_array(ps.bits) for ps in self.passes]
         self.rotmask = [sum(1 << a for a, b in enumerate(ps.bits) if b in ps.rot) for ps in self.passes]
-        self.psi = torch.empty((2, cnt, self.dim), dtype=mats.dtype, device=device)
+        self.psi = psi.view(2, cnt, self.dim)
         self.mats = mats.view(self.lmax, len(self.passes), cnt, self.width, 1, 4)
-        self.sel = []
-        for layer in range(self.lmax):
-            active = np.nonzero(self.layers > layer)[0]
-            self.sel.append(None if len(active) == cnt else torch.tensor(active, dtype=torch.int32, device=device))
         self.nsel = [int(np.sum(self.layers > layer)) for layer in range(self.lmax)]
         final_buf = (self.layers - 1) % 2
         self.tfim_sel = torch.tensor(final_buf * cnt + np.arange(cnt), dtype=torch.int32, device=device)
@@ -95,11 +120,23 @@ class _PassGroup:
         self.partials = torch.zeros((cnt, self.tfim_cols), dtype=torch.float64, device=device)
         self.cols = [int(min(self.dim >> TILE_BITS, 65535)) if ps.kind == "tile"
                      else int(min(-(-(self.dim >> len(ps.bits)) // ROT_BLOCK), 65535)) for ps in self.passes]
+        self.steps = self.passes[0].kind == "step"
 
-    def launch(self, code, g, stream, energies_out):
+    def step_entry(self, t, first_state, first_slot):
+        """Entry of ``qj_ansatz_step`` for this group's t-th pass."""
+        layer, i = divmod(t, len(self.passes))
+        half = self.cnt * self.dim
+        dst = first_state + (layer % 2) * half
+        src = dst if i else -1 if layer == 0 else first_state + ((layer - 1) % 2) * half
+        bits = list(self.passes[i].bits)
+        ka = min(5, len(bits))
+        slot = first_slot + (layer * len(self.passes) + i) * self.cnt * self.width
+        return [self.n, self.nsel[layer], src, dst, int(i == 0 and layer > 0), slot, self.width, ka, len(bits) - ka,
+                *bits, *[0] * (STEP_BITS - len(bits))]
+
+    def launch_passes(self, code, stream):
         psi = self.psi
         for layer in range(self.lmax):
-            sel = self.sel[layer]
             for i, (bits_ptr, _keep, nbits) in enumerate(self.bits):
                 if layer == 0 and i == 0:
                     src, dst, load = None, psi[0], LOAD_ZERO
@@ -108,14 +145,16 @@ class _PassGroup:
                 else:
                     src, dst, load = psi[layer % 2], psi[layer % 2], LOAD_PLAIN
                 if self.passes[i].kind == "tile":
-                    call("qj_rot_tile_pass", _vp(src), _vp(dst), None, None, code, self.n, self.dim, _vp(sel),
+                    call("qj_rot_tile_pass", _vp(src), _vp(dst), None, None, code, self.n, self.dim, None,
                          self.nsel[layer], bits_ptr, self.rotmask[i], 1, None, load, _vp(self.mats[layer, i]),
                          self.width * 4, None, self.cols[i], stream)
                 else:
-                    call("qj_rot_pass", _vp(src), _vp(dst), None, None, code, self.n, self.dim, _vp(sel),
+                    call("qj_rot_pass", _vp(src), _vp(dst), None, None, code, self.n, self.dim, None,
                          self.nsel[layer], bits_ptr, nbits, 1, None, load, _vp(self.mats[layer, i]),
                          self.width * 4, None, self.cols[i], stream)
-        call("qj_tfim_batch", _vp(psi), None, code, self.n, self.dim, _vp(self.tfim_sel), self.cnt, g, 1,
+
+    def launch_energies(self, code, g, stream, energies_out):
+        call("qj_tfim_batch", _vp(self.psi), None, code, self.n, self.dim, _vp(self.tfim_sel), self.cnt, g, 1,
              _vp(self.partials), self.tfim_cols, stream)
         call("qj_reduce_rows", _vp(self.partials), self.cnt, self.tfim_cols, _vp(energies_out), stream)
 
@@ -134,7 +173,9 @@ class AnsatzBatch:
         self.device = torch.device("cuda", 0) if device is None else torch.device(device)
         ncirc = len(self.shapes)
         nq = np.array([s[0] for s in self.shapes])
-        self.order = np.argsort(nq, kind="stable")  # sorted position -> circuit
+        depth = np.array([s[1] for s in self.shapes])
+        # sorted position -> circuit: by qubits, then by descending layers
+        self.order = np.lexsort((-depth, nq))
         self.inv = torch.from_numpy(np.argsort(self.order)).to(self.device)
         self.plan = dict(plan) if plan is not None else default_plan(sorted(set(nq.tolist())), self.tdtype)
         for n in set(nq.tolist()):
@@ -186,10 +227,10 @@ class AnsatzBatch:
             members = [c for c in self.order[self.nlds:] if self.shapes[c][0] == n]
             layers = [self.shapes[c][1] for c in members]
             k = None if self.plan[n][0] == "tile" else self.plan[n][1]
-            passes = _passes(n, k)
+            passes = _passes(n, k, self.tdtype)
             width = max(len(ps.bits) for ps in passes)
             per_layer = len(passes) * len(members) * width
-            groups.append((n, members, layers, k, at, per_layer * max(layers)))
+            groups.append((n, members, layers, passes, at, per_layer * max(layers)))
             recs += [(poffs[c], at + s * width, n, nl, per_layer, len(slots))
                      for s, (c, nl) in enumerate(zip(members, layers))]
             slots += pass_slots(passes, len(members), width)
@@ -199,13 +240,23 @@ class AnsatzBatch:
         self.mat_recs = torch.tensor(np.array(recs, dtype=np.int64), device=self.device)
         self.mat_slots = torch.tensor(slots, dtype=torch.int32, device=self.device)
         self.lds_mats = self.mats[: sum(self.shapes[c][0] * self.shapes[c][1] for c in self.order[: self.nlds])]
+        self.states = torch.empty(sum(2 * len(grp[1]) << grp[0] for grp in groups), dtype=self.tdtype,
+                                  device=self.device)
         self.pass_groups = []
-        pos = self.nlds
-        for n, members, layers, k, first_slot, count in groups:
-            grp = _PassGroup(n, members, layers, k, self.mats[first_slot: first_slot + count], self.device)
+        pos, first_state, entries = self.nlds, 0, []
+        for n, members, layers, passes, first_slot, count in groups:
+            size = 2 * len(members) << n
+            grp = _PassGroup(n, members, layers, passes, self.states[first_state: first_state + size],
+                             self.mats[first_slot: first_slot + count], self.device)
             grp.offset = pos
             pos += len(members)
             self.pass_groups.append(grp)
+            if grp.steps:
+                for t in range(grp.lmax * len(passes)):
+                    entries += [[]] * (t + 1 - len(entries))
+                    entries[t] = [grp.step_entry(t, first_state, first_slot)] + entries[t]  # largest first
+            first_state += size
+        self.steps = [(len(rows), np.array(rows, dtype=np.int64)) for rows in entries]
         self.graph = None
 
     # -------------------------------------------------------------- data --
@@ -236,9 +287,14 @@ class AnsatzBatch:
         if self.nlds:
             call("qj_ansatz_lds", self.code, _vp(self.lds_desc), self.nlds, _vp(self.lds_mats), self.lds_mats.numel(),
                  self.g, _vp(self.energies_sorted), self.lds_nqmax, self.lds_blocks, stream)
+        for count, rows in self.steps:
+            call("qj_ansatz_step", _vp(self.states), self.code, self.states.numel(), _vp(self.mats),
+                 self.mats.numel(), ctypes.c_void_p(rows.ctypes.data), count, stream)
         for grp in self.pass_groups:
+            if not grp.steps:
+                grp.launch_passes(self.code, stream)
             out = self.energies_sorted[grp.offset: grp.offset + grp.cnt]
-            grp.launch(self.code, self.g, stream, out)
+            grp.launch_energies(self.code, self.g, stream, out)
 
     def capture(self):
         """Record ``run`` into one graph (after an eager warm-up)."""

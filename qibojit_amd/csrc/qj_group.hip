@@ -839,6 +839,158 @@ __global__ void __launch_bounds__(kTileBlock)
   }
 }
 
+// --------------------------------------------- layers of many circuits --
+// One step of every circuit of a batch too large for LDS, in one launch: entry
+// e rotates ka + kb <= 10 bits (in the given order) of `count` states of n >= 12
+// qubits.  A workgroup of 128 threads owns one tile of 2^12 amplitudes: the
+// rotated bits and the lowest others.  Each thread holds 32 amplitudes: the
+// first ka bits are rotated on registers (layout A: register bits a[0..4]),
+// the tile goes through LDS, the next kb on registers again (layout B).  Every
+// amplitude meets its rotations in the order of the bits, as in one register
+// pass per group, so the results are the same to the bit.  LDS index of an
+// amplitude: f | (b ^ a) << 2 | a << 7 (f: the two bits in neither register
+// set), which keeps both the writes (lanes f, b) and the reads (lanes f, a) of a
+// wave on different banks.
+// Register passes of one group each moved every state once per 5 bits and ran
+// qubit count after qubit count, with 30 workgroups at 14 qubits: 3.5 ms in 254
+// launches for the passes of 192 circuits of 8 to 20 qubits, 2 to 10 layers.
+// Now 1.5 ms in 20 launches, at about 4 TB/s, which bounds it.
+constexpr int kStepBits = 12, kStepRegs = 5, kStepBlock = 128, kStepEntries = 24;
+
+struct StepEntry {
+  u64 src, dst;       // first state's offset; src == ~0: |0...0>
+  u64 mats, mstride;  // first state's matrices, in numbers
+  unsigned first;     // first workgroup
+  int n, ka, kb, ladder;
+  unsigned char a[kStepRegs], b[kStepRegs], f[2];  // positions
+  unsigned char la[7], lb[7];                      // lane positions, ascending
+  unsigned char ia[7], ib[7];                      // what lane bit i is: LDS index bit of that layout
+  unsigned char tile[kStepBits];                   // all positions, ascending
+};
+struct StepArgs {
+  int count;
+  StepEntry e[kStepEntries];
+};
+
+// m * x with the roundings that the compiler gives the products of rot_apply.
+template <typename R>
+__device__ __forceinline__ cplx<R> step_mul(cplx<R> m, cplx<R> x) {
+  return mk<R>(rfma(m.re, x.re, -(m.im * x.im)), rfma(m.re, x.im, m.im * x.re));
+}
+
+template <typename R, int A>
+__device__ __forceinline__ void step_rotate(cplx<R> (&x)[32], const cplx<R>* m, int count) {
+  if constexpr (A < kStepRegs) {
+    if (A < count) {
+      const cplx<R> m00 = m[4 * A], m01 = m[4 * A + 1], m10 = m[4 * A + 2], m11 = m[4 * A + 3];
+#pragma unroll
+      for (int r = 0; r < 32; ++r) {
+        if (r & (1 << A)) continue;
+        const cplx<R> a = x[r], b = x[r | (1 << A)];
+        x[r] = cadd(step_mul(m00, a), step_mul(m01, b));
+        x[r | (1 << A)] = cadd(step_mul(m10, a), step_mul(m11, b));
+      }
+      step_rotate<R, A + 1>(x, m, count);
+    }
+  }
+}
+
+template <typename R>
+__global__ void __launch_bounds__(kStepBlock, 2) k_ansatz_step(cplx<R>* states, const cplx<R>* mats, StepArgs a) {
+  __shared__ __align__(16) cplx<R> sm[1 << kStepBits];
+  int k = 0;
+  while (k + 1 < a.count && blockIdx.x >= a.e[k + 1].first) ++k;
+  const StepEntry& e = a.e[k];
+  const unsigned local = blockIdx.x - e.first;
+  const unsigned row = local >> (e.n - kStepBits);
+  u64 base = local & ((1u << (e.n - kStepBits)) - 1);
+#pragma unroll
+  for (int j = 0; j < kStepBits; ++j) {
+    const u64 lo = base & ((u64(1) << e.tile[j]) - 1);
+    base = ((base ^ lo) << 1) | lo;
+  }
+  const unsigned tid = threadIdx.x;
+  u64 lane_a = 0, lane_b = 0;
+  unsigned at_a = 0, at_b = 0;
+#pragma unroll
+  for (int i = 0; i < 7; ++i) {
+    const u64 on = (tid >> i) & 1;
+    lane_a |= on << e.la[i];
+    lane_b |= on << e.lb[i];
+    at_a ^= (unsigned)on << e.ia[i];
+    at_b ^= (unsigned)on << e.ib[i];
+  }
+  at_b ^= at_b >> 7 << 2;  // layout B's lanes hold a
+  u64 off[kStepRegs];
+#pragma unroll
+  for (int i = 0; i < kStepRegs; ++i) off[i] = u64(1) << e.a[i];
+  cplx<R> x[32];
+  const u64 in = base | lane_a;
+  const bool pairs = e.a[0] == 0;  // registers 2r, 2r + 1 are neighbours
+  if (e.src == ~u64(0)) {
+#pragma unroll
+    for (int r = 0; r < 32; ++r) x[r] = mk<R>(R(in == 0 && r == 0 ? 1 : 0), R(0));
+  } else {
+    const cplx<R>* p = states + e.src + ((u64)row << e.n);
+#pragma unroll
+    for (int r = 0; r < 32; r += 2) {
+      u64 k0 = in;
+#pragma unroll
+      for (int i = 1; i < kStepRegs; ++i)
+        if ((r >> i) & 1) k0 |= off[i];
+      if (pairs) {
+        const u64 s0 = e.ladder ? k0 ^ (k0 >> 1) : k0;
+        const cvec<R, 2> v = ldv<R, 2>(p + (s0 & ~u64(1)));
+        const bool sw = s0 & 1;
+        x[r] = sw ? v.v[1] : v.v[0];
+        x[r + 1] = sw ? v.v[0] : v.v[1];
+      } else {
+        const u64 k1 = k0 | off[0];
+        x[r] = p[e.ladder ? k0 ^ (k0 >> 1) : k0];
+        x[r + 1] = p[e.ladder ? k1 ^ (k1 >> 1) : k1];
+      }
+    }
+  }
+  const cplx<R>* m = mats + e.mats + row * e.mstride;
+  step_rotate<R, 0>(x, m, e.ka);
+  cplx<R>* out = states + e.dst + ((u64)row << e.n);
+  if (e.kb == 0) {
+#pragma unroll
+    for (int r = 0; r < 32; r += 2) {
+      u64 k0 = in;
+#pragma unroll
+      for (int i = 1; i < kStepRegs; ++i)
+        if ((r >> i) & 1) k0 |= off[i];
+      if (pairs) {
+        cvec<R, 2> v;
+        v.v[0] = x[r];
+        v.v[1] = x[r + 1];
+        stv<R, 2>(out + k0, v);
+      } else {
+        out[k0] = x[r];
+        out[k0 | off[0]] = x[r + 1];
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < 32; ++r) sm[(at_a ^ (r << 2)) | (r << 7)] = x[r];
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 32; ++r) x[r] = sm[at_b ^ (r << 2)];
+  step_rotate<R, 0>(x, m + 4 * e.ka, e.kb);
+#pragma unroll
+  for (int i = 0; i < kStepRegs; ++i) off[i] = u64(1) << e.b[i];
+#pragma unroll
+  for (int r = 0; r < 32; ++r) {
+    u64 k0 = base | lane_b;
+#pragma unroll
+    for (int i = 0; i < kStepRegs; ++i)
+      if ((r >> i) & 1) k0 |= off[i];
+    out[k0] = x[r];
+  }
+}
+
 // ------------------------------------------------ whole circuit in LDS --
 // Persistent kernel for small ansatz circuits: workgroup w runs circuits
 // w, w + gridDim.x, ... entirely in LDS (2^n amplitudes, n <= nqmax) and
@@ -1263,6 +1415,95 @@ int qj_ansatz_mats(const double* params, uint64_t nparams, const int64_t* recs, 
   else
     return set_error(QJ_EVALUE, "ansatz_mats: dtype must be complex64/complex128");
   return check_launch("ansatz_mats launch");
+}
+
+int qj_ansatz_step(void* states, int dtype, uint64_t states_len, const void* mats, uint64_t mats_len,
+                   const int64_t* entries, int nentries, void* stream) {
+  if (!states || !mats || !entries) return set_error(QJ_EVALUE, "ansatz_step: null pointer");
+  if (nentries < 0 || nentries > kStepEntries)
+    return set_error(QJ_EVALUE, "ansatz_step: %d entries (at most %d)", nentries, kStepEntries);
+  if (nentries == 0) return QJ_OK;
+  if ((reinterpret_cast<uintptr_t>(states) & 31) != 0)
+    return set_error(QJ_EVALUE, "ansatz_step: states must be 32-byte aligned");
+  StepArgs a{};
+  a.count = nentries;
+  u64 blocks = 0;
+  for (int k = 0; k < nentries; ++k) {
+    const int64_t* r = entries + (size_t)k * QJ_STEP_WORDS;
+    StepEntry& e = a.e[k];
+    const int64_t n = r[0], count = r[1], src = r[2], dst = r[3], ka = r[7], kb = r[8];
+    if (n < kStepBits || n > 40) return set_error(QJ_EVALUE, "ansatz_step: %lld qubits", (long long)n);
+    if (count < 1 || count > (1 << 20)) return set_error(QJ_EVALUE, "ansatz_step: %lld states", (long long)count);
+    const u64 len = (u64)count << n;
+    if (len > states_len || dst < 0 || (u64)dst > states_len - len || src < -1 ||
+        (src >= 0 && (u64)src > states_len - len) || (dst | (src < 0 ? 0 : src)) & 1)
+      return set_error(QJ_EVALUE, "ansatz_step: states out of range");
+    if (src >= 0 && (r[4] || src != dst) && (u64)(src > dst ? src - dst : dst - src) < len)
+      return set_error(QJ_EVALUE, "ansatz_step: states overlap");
+    if (ka < 1 || ka > kStepRegs || kb < 0 || kb > kStepRegs)
+      return set_error(QJ_EVALUE, "ansatz_step: bad bit counts %lld, %lld", (long long)ka, (long long)kb);
+    const int64_t mlen = (int64_t)(mats_len / 4);
+    if (r[5] < 0 || r[5] > mlen || r[6] < 0 || r[6] > mlen || r[5] + (count - 1) * r[6] + ka + kb > mlen)
+      return set_error(QJ_EVALUE, "ansatz_step: matrices out of range");
+    u64 used = 0;
+    for (int i = 0; i < ka + kb; ++i) {
+      const int64_t bit = r[9 + i];
+      if (bit < 0 || bit >= n || (used >> bit) & 1) return set_error(QJ_EVALUE, "ansatz_step: bad bit");
+      used |= u64(1) << bit;
+      (i < ka ? e.a[i] : e.b[i - ka]) = (unsigned char)bit;
+    }
+    // the lowest other bits complete the tile: the highest of them fill the
+    // register sets, so that lanes keep the low ones
+    unsigned char fill[kStepBits];
+    int nfill = 0;
+    for (int bit = 0; nfill < kStepBits - ka - kb; ++bit)
+      if (!((used >> bit) & 1)) fill[nfill++] = (unsigned char)bit;
+    for (int i = 0; i < nfill; ++i) used |= u64(1) << fill[i];
+    for (int i = (int)ka; i < kStepRegs; ++i) e.a[i] = fill[--nfill];
+    for (int i = (int)kb; i < kStepRegs; ++i) e.b[i] = fill[--nfill];
+    e.f[0] = fill[0];
+    e.f[1] = fill[1];
+    int nt = 0, na = 0, nb = 0;
+    for (int bit = 0; bit < n; ++bit) {
+      if (!((used >> bit) & 1)) continue;
+      e.tile[nt++] = (unsigned char)bit;
+      int where = -1;  // its LDS index bit
+      for (int i = 0; i < kStepRegs; ++i) {
+        if (e.a[i] == bit) where = 7 + i;
+        if (e.b[i] == bit) where = 2 + i;
+      }
+      for (int i = 0; i < 2; ++i)
+        if (e.f[i] == bit) where = i;
+      if (where < 7) {
+        e.la[na] = (unsigned char)bit;
+        e.ia[na++] = (unsigned char)where;
+      }
+      if (where < 2 || where >= 7) {
+        e.lb[nb] = (unsigned char)bit;
+        e.ib[nb++] = (unsigned char)where;
+      }
+    }
+    e.n = (int)n;
+    e.ka = (int)ka;
+    e.kb = (int)kb;
+    e.ladder = r[4] != 0;
+    e.src = src < 0 ? ~u64(0) : (u64)src;
+    e.dst = (u64)dst;
+    e.mats = (u64)r[5] * 4;
+    e.mstride = (u64)r[6] * 4;
+    e.first = (unsigned)blocks;
+    blocks += (u64)count << (n - kStepBits);
+    if (blocks > 0x7fffffffull) return set_error(QJ_EVALUE, "ansatz_step: too many tiles");
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 gd((unsigned)blocks), bd(kStepBlock);
+  if (dtype == QJ_COMPLEX64)
+    k_ansatz_step<float><<<gd, bd, 0, st>>>((cplx<float>*)states, (const cplx<float>*)mats, a);
+  else if (dtype == QJ_COMPLEX128)
+    k_ansatz_step<double><<<gd, bd, 0, st>>>((cplx<double>*)states, (const cplx<double>*)mats, a);
+  else
+    return set_error(QJ_EVALUE, "ansatz_step: dtype must be complex64/complex128");
+  return check_launch("ansatz_step launch");
 }
 
 int qj_reduce_rows(const double* in, uint64_t nrows, uint64_t ncols, double* out, void* stream) {
