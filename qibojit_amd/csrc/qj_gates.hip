@@ -32,6 +32,17 @@ struct M2 {
   cplx<R> m[16];
 };
 
+// Matrices of up to three targets are kernel arguments (at most 1 KiB): a copy
+// to the device and its event in front of the launch cost a 10-qubit call 3-6 us
+// on the host and a dispatch of their own: 48 gates on 10 qubits, one call each,
+// went from 669 to 538 us.  Lanes that need different entries load them from the
+// argument block; rows read by scalar loads and picked with selects cost
+// two-target gates on 30 complex64 qubits 2.5% and three-target ones up to 5%.
+template <typename R, int N>
+struct MatArg {
+  cplx<R> m[N];
+};
+
 // One work item per thread and a full grid: measured fastest on gfx950 for
 // every target stride (more items per thread or a persistent grid lowered
 // the in-place rate by 5-10%).
@@ -147,8 +158,9 @@ __global__ void __launch_bounds__(NT)
 }
 
 // ------------------------------------------------------ 3..5 qubits (regs) --
-// The 2^K amplitudes of a group are held in registers; the matrix is staged
-// once per workgroup in LDS and read as wave-uniform broadcasts.
+// The 2^K amplitudes of a group are held in registers; the matrix (3 targets: a
+// kernel argument) is staged once per workgroup in LDS and read as wave-uniform
+// broadcasts.
 template <int K>
 struct Offs {
   u64 o[1 << K];
@@ -157,8 +169,9 @@ struct Offs {
 template <typename R, int K, int NT = kBlock>
 __global__ void __launch_bounds__(NT)
     k_multi_reg(cplx<R>* __restrict__ st, u64 ngroups, Ins ins, Offs<K> off,
-                const cplx<R>* __restrict__ mat) {
+                const cplx<R>* __restrict__ mat, MatArg<R, K == 3 ? 64 : 1> arg) {
   constexpr int N = 1 << K;
+  constexpr bool kArg = K == 3;
   __shared__ cplx<R> sm[N * N];
   const u64 stride = (u64)gridDim.x * NT;
   u64 g = (u64)blockIdx.x * NT + threadIdx.x;
@@ -172,7 +185,7 @@ __global__ void __launch_bounds__(NT)
 #pragma unroll
     for (int c = 0; c < N; ++c) x[c] = st[base + off.o[c]];
   }
-  for (int t = threadIdx.x; t < N * N; t += NT) sm[t] = mat[t];
+  for (int t = threadIdx.x; t < N * N; t += NT) sm[t] = kArg ? arg.m[t] : mat[t];
   __syncthreads();
   for (; g < ngroups; g += stride) {
 #pragma unroll 1
@@ -260,7 +273,7 @@ __device__ __forceinline__ cplx<R> shfl_xor_c(cplx<R> a, int mask) {
 // ILP chunks per wave and loop step (QJ_WAVE_ILP = 1 (default), 2, 4).
 template <typename R, int K, int ILP>
 __global__ void __launch_bounds__(kBlock)
-    k_wave(cplx<R>* __restrict__ st, u64 nchunks, Ins ins, WaveSpec<K> ws, const cplx<R>* __restrict__ mat) {
+    k_wave(cplx<R>* __restrict__ st, u64 nchunks, Ins ins, WaveSpec<K> ws, MatArg<R, 1 << (2 * K)> mat) {
   constexpr int N = 1 << K;
   const int lane = threadIdx.x & 63;
   int r = 0;
@@ -268,7 +281,7 @@ __global__ void __launch_bounds__(kBlock)
   for (int u = 0; u < K; ++u) r |= ((lane >> ws.tb[u]) & 1) << (K - 1 - u);
   cplx<R> row[N];
 #pragma unroll
-  for (int c = 0; c < N; ++c) row[c] = mat[r * N + c];
+  for (int c = 0; c < N; ++c) row[c] = mat.m[r * N + c];
   const bool store = (lane & ws.cmask) == ws.cones;
   const u64 wave = (u64)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   const u64 nwaves = (u64)gridDim.x * (kBlock / 64);
@@ -317,11 +330,11 @@ __global__ void __launch_bounds__(kBlock)
 // zero terms of the dense row change nothing but the sign of a zero sum).
 template <typename R, int ILP>
 __global__ void __launch_bounds__(kBlock)
-    k_wave_pair(cplx<R>* __restrict__ st, u64 nchunks, Ins ins, WaveSpec<2> ws, const cplx<R>* __restrict__ mat) {
+    k_wave_pair(cplx<R>* __restrict__ st, u64 nchunks, Ins ins, WaveSpec<2> ws, MatArg<R, 16> mat) {
   const int lane = threadIdx.x & 63;
   const int r = (((lane >> ws.tb[0]) & 1) << 1) | ((lane >> ws.tb[1]) & 1);
   const int rp = r ^ 3;
-  const cplx<R> cs = mat[r * 4 + r], cp = mat[r * 4 + rp];
+  const cplx<R> cs = mat.m[r * 4 + r], cp = mat.m[r * 4 + rp];
   const bool self_first = r < rp;
   const int xm = ws.xmask[3];
   const bool store = (lane & ws.cmask) == ws.cones;
@@ -359,16 +372,11 @@ __global__ void __launch_bounds__(kBlock)
 // distinct 16-byte bank groups within every 8 lanes.
 constexpr int kLow3Chunk = 2048;
 
-template <typename R>
-constexpr size_t mat_bytes_of(int n) {
-  return (size_t)n * n * sizeof(cplx<R>);
-}
-
 __device__ __forceinline__ unsigned low3_swz(unsigned s) { return s ^ ((s >> 3) & 7u); }
 
 template <typename R, int CHUNK>
 __global__ void __launch_bounds__(CHUNK / 8)
-    k_multi_low3(cplx<R>* __restrict__ st, u64 nchunks, Offs32 roff, const cplx<R>* __restrict__ mat) {
+    k_multi_low3(cplx<R>* __restrict__ st, u64 nchunks, Offs32 roff, MatArg<R, 64> mat) {
   constexpr int NT = CHUNK / 8;  // one 8-amplitude group per thread
   __shared__ cplx<R> buf[CHUNK];
   const unsigned t = threadIdx.x;
@@ -382,9 +390,9 @@ __global__ void __launch_bounds__(CHUNK / 8)
     for (int r = 0; r < 8; ++r) x[r] = buf[low3_swz(8 * t + (unsigned)roff.o[r])];
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      cplx<R> acc = cmul(mat[r * 8], x[0]);
+      cplx<R> acc = cmul(mat.m[r * 8], x[0]);
 #pragma unroll
-      for (int k = 1; k < 8; ++k) acc = cadd(acc, cmul(mat[r * 8 + k], x[k]));
+      for (int k = 1; k < 8; ++k) acc = cadd(acc, cmul(mat.m[r * 8 + k], x[k]));
       buf[low3_swz(8 * t + (unsigned)roff.o[r])] = acc;
     }
     __syncthreads();
@@ -452,11 +460,6 @@ static int try_wave(cplx<R>* st, int nqubits, const int* tb, int k, const Ins& g
   }
   ins.npos = nh;
   const u64 nchunks = u64(1) << (nqubits - kWaveBits - nh);
-  const int N = 1 << k;
-  void* dmat = nullptr;
-  int ticket = -1;
-  *rc = ring_upload(dense, (size_t)N * N * sizeof(cplx<R>), s, &dmat, &ticket);
-  if (*rc) return 1;
   // chunks per wave step: QJ_WAVE_ILP overrides; by default 1 for complex128
   // (16-byte lanes; 5.9 vs 5.6 TB/s with 2 at 30 qubits) and 2 for complex64
   // (8-byte lanes need more loads in flight)
@@ -468,9 +471,10 @@ static int try_wave(cplx<R>* st, int nqubits, const int* tb, int k, const Ins& g
   const int ilp = ilp_env ? ilp_env : (sizeof(R) == 4 ? 2 : 1);
   const u64 waves = (nchunks + ilp - 1) / ilp;
   const u64 grid = grid_for(waves, kBlock / 64);
-  const cplx<R>* dm = static_cast<const cplx<R>*>(dmat);
 #define QJ_WAVE(KK)                                                                 \
   {                                                                                 \
+    MatArg<R, 1 << (2 * KK)> dm;                                                    \
+    std::memcpy(dm.m, dense, sizeof(dm.m));                                         \
     WaveSpec<KK> ws;                                                                \
     for (int u = 0; u < KK; ++u) ws.tb[u] = tb[u];                                  \
     for (int d = 0; d < (1 << KK); ++d) {                                           \
@@ -493,6 +497,8 @@ static int try_wave(cplx<R>* st, int nqubits, const int* tb, int k, const Ins& g
     for (int c = 0; c < 4; ++c)
       if (c != r && c != (r ^ 3) && (dense[r * 4 + c].re != 0 || dense[r * 4 + c].im != 0)) pair = false;
   if (pair) {
+    MatArg<R, 16> dm;
+    std::memcpy(dm.m, dense, sizeof(dm.m));
     WaveSpec<2> ws;
     ws.tb[0] = tb[0];
     ws.tb[1] = tb[1];
@@ -505,7 +511,6 @@ static int try_wave(cplx<R>* st, int nqubits, const int* tb, int k, const Ins& g
   } else if (k == 1) QJ_WAVE(1) else QJ_WAVE(2)
 #undef QJ_WAVE
   *rc = check_launch("wave gate launch");
-  ring_release(ticket, s);
   return 1;
 }
 
@@ -689,7 +694,9 @@ static int two_qubit_impl(void* state, int nqubits, int kind, int bit1, int bit2
 
 template <typename R, int K>
 static void launch_multi_reg(cplx<R>* st, u64 ngroups, const Ins& ins, const int* tb,
-                             const cplx<R>* dmat, hipStream_t s) {
+                             const cplx<R>* dmat, const cplx<R>* gate, hipStream_t s) {
+  MatArg<R, K == 3 ? 64 : 1> arg;
+  std::memcpy(arg.m, gate, sizeof(arg.m));
   Offs<K> off;
   for (int r = 0; r < (1 << K); ++r) {
     u64 o = 0;
@@ -716,11 +723,11 @@ static void launch_multi_reg(cplx<R>* st, u64 ngroups, const Ins& ins, const int
   if (nt_env) nt = nt_env;
   const u64 grid = grid_for(ngroups, (u64)nt);
   if (nt == 128)
-    k_multi_reg<R, K, 128><<<dim3((unsigned)grid), dim3(128), 0, s>>>(st, ngroups, ins, off, dmat);
+    k_multi_reg<R, K, 128><<<dim3((unsigned)grid), dim3(128), 0, s>>>(st, ngroups, ins, off, dmat, arg);
   else if (nt == 512)
-    k_multi_reg<R, K, 512><<<dim3((unsigned)grid), dim3(512), 0, s>>>(st, ngroups, ins, off, dmat);
+    k_multi_reg<R, K, 512><<<dim3((unsigned)grid), dim3(512), 0, s>>>(st, ngroups, ins, off, dmat, arg);
   else
-    k_multi_reg<R, K><<<dim3((unsigned)grid), dim3(kBlock), 0, s>>>(st, ngroups, ins, off, dmat);
+    k_multi_reg<R, K><<<dim3((unsigned)grid), dim3(kBlock), 0, s>>>(st, ngroups, ins, off, dmat, arg);
 }
 
 template <typename R>
@@ -753,10 +760,6 @@ static int multi_qubit_impl(void* state, int nqubits, const int32_t* target_bits
           if ((r >> (2 - u)) & 1) o |= u64(1) << tb[u];
         roff.o[r] = o;
       }
-      void* dmat = nullptr;
-      int ticket = -1;
-      rc = ring_upload(gate, mat_bytes_of<R>(8), s, &dmat, &ticket);
-      if (rc) return rc;
       static const int chunk_env = [] {
         const char* e = std::getenv("QJ_LOW3_CHUNK");
         const int v = e ? std::atoi(e) : 0;
@@ -767,19 +770,23 @@ static int multi_qubit_impl(void* state, int nqubits, const int32_t* target_bits
       const int dflt = sizeof(R) == 8 ? 1024 : kLow3Chunk;
       const int chunk = (chunk_env && (u64(1) << nqubits) >= (u64)chunk_env) ? chunk_env : dflt;
       const u64 nchunks = (u64(1) << nqubits) / (u64)chunk;
-      const cplx<R>* dm = static_cast<const cplx<R>*>(dmat);
+      MatArg<R, 64> dm;
+      std::memcpy(dm.m, gate, sizeof(dm.m));
       if (chunk == 1024)
         k_multi_low3<R, 1024><<<dim3((unsigned)grid_for(nchunks, 1)), dim3(128), 0, s>>>(st, nchunks, roff, dm);
       else if (chunk == 4096)
         k_multi_low3<R, 4096><<<dim3((unsigned)grid_for(nchunks, 1)), dim3(512), 0, s>>>(st, nchunks, roff, dm);
       else
         k_multi_low3<R, 2048><<<dim3((unsigned)grid_for(nchunks, 1)), dim3(256), 0, s>>>(st, nchunks, roff, dm);
-      rc = check_launch("apply_multi_qubit launch");
-      ring_release(ticket, s);
-      return rc;
+      return check_launch("apply_multi_qubit launch");
     }
   }
 
+  const cplx<R>* host = static_cast<const cplx<R>*>(gate);
+  if (K == 3) {
+    launch_multi_reg<R, 3>(st, ngroups, ins, tb.data(), nullptr, host, s);
+    return check_launch("apply_multi_qubit launch");
+  }
   const size_t mat_bytes = (size_t)N * N * sizeof(cplx<R>);
   if (K <= 5) {
     void* dmat = nullptr;
@@ -787,9 +794,8 @@ static int multi_qubit_impl(void* state, int nqubits, const int32_t* target_bits
     rc = ring_upload(gate, mat_bytes, s, &dmat, &ticket);
     if (rc) return rc;
     const cplx<R>* dm = static_cast<const cplx<R>*>(dmat);
-    if (K == 3) launch_multi_reg<R, 3>(st, ngroups, ins, tb.data(), dm, s);
-    else if (K == 4) launch_multi_reg<R, 4>(st, ngroups, ins, tb.data(), dm, s);
-    else launch_multi_reg<R, 5>(st, ngroups, ins, tb.data(), dm, s);
+    if (K == 4) launch_multi_reg<R, 4>(st, ngroups, ins, tb.data(), dm, host, s);
+    else launch_multi_reg<R, 5>(st, ngroups, ins, tb.data(), dm, host, s);
     rc = check_launch("apply_multi_qubit launch");
     ring_release(ticket, s);
     return rc;
