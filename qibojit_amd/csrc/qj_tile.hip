@@ -40,6 +40,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "qj_common.h"
@@ -49,6 +50,14 @@ namespace qj {
 
 constexpr int kTileMaxHighBits = 12;  // QJ_TILE_MAX_BITS - 1 (one low bit at least)
 constexpr int kTileLA = 8;  // tile bits indexing phase table A
+// A register kernel's plan of up to 3.5 KiB (4 KiB of arguments less the others)
+// travels with the launch: its copy to the device, a dispatch and an event of
+// their own, cost a pass of a 20-qubit circuit (24 gates, 31 us) 7 us.  The
+// 20-qubit random circuit of depth 20 went from 1.07 to 0.87 ms.
+struct PlanArg {
+  alignas(16) char data[3584];
+};
+struct NoPlan {};
 
 struct TileSpec {
   int L;                       // low contiguous bits
@@ -336,10 +345,15 @@ __device__ __forceinline__ u64 uni64(u64 v) {
 // thread each, double-buffered by tile parity), the loads, and the ops of
 // every segment; plan values read from LDS are made wave-uniform so the op
 // dispatch is scalar.  WPE: waves per SIMD the register budget must allow.
-template <typename R, int NRB, int BSMAX, int WPE>
+// Plan: PlanArg when the plan fits the kernel's arguments (it is the first one,
+// so it is read through the argument segment's own pointer: a pointer to the
+// parameter would be a per-thread copy), NoPlan when it is at plan_buf.
+template <typename R, int NRB, int BSMAX, int WPE, typename Plan>
 __global__ void __launch_bounds__(BSMAX, WPE)
-    k_tile_reg(const cplx<R>* src, cplx<R>* st, u64 ntiles, Ins tins, const char* __restrict__ plan) {
+    k_tile_reg(Plan, const cplx<R>* src, cplx<R>* st, u64 ntiles, Ins tins, const char* __restrict__ plan_buf) {
   constexpr int NR = 1 << NRB;
+  const char* plan = plan_buf;
+  if constexpr (std::is_same<Plan, PlanArg>::value) plan = (const char*)__builtin_amdgcn_kernarg_segment_ptr();
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   const RegHead& h = *reinterpret_cast<const RegHead*>(plan);
   const int TB = h.TB, NT = h.NT, nseg = h.nseg, nphase = h.nphase, ga = h.ga;
@@ -689,30 +703,30 @@ static int tile_register_bits(bool dbl, int maxk) {
   return nrb <= hi ? nrb : 0;
 }
 
-template <typename R, int NRB, int BSMAX, int WPE>
+template <typename R, int NRB, int BSMAX, int WPE, typename Plan>
 static void launch_reg(dim3 gd, dim3 bd, size_t lds, hipStream_t s, const cplx<R>* src, cplx<R>* st, u64 ntiles,
-                       const Ins& tins, const char* plan) {
+                       const Ins& tins, const Plan& arg, const char* plan) {
   // dynamic LDS above 64 KiB needs the kernel's limit raised first
   if (lds > 65536)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tile_reg<R, NRB, BSMAX, WPE>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tile_reg<R, NRB, BSMAX, WPE, Plan>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  k_tile_reg<R, NRB, BSMAX, WPE><<<gd, bd, lds, s>>>(src, st, ntiles, tins, plan);
+  k_tile_reg<R, NRB, BSMAX, WPE><<<gd, bd, lds, s>>>(arg, src, st, ntiles, tins, plan);
 }
 
-template <typename R>
+template <typename R, typename Plan>
 static void launch_tile_reg(int nrb, int NT, u64 grid, size_t lds, hipStream_t s, const cplx<R>* src, cplx<R>* st,
-                            u64 ntiles, const Ins& tins, const char* plan) {
+                            u64 ntiles, const Ins& tins, const Plan& arg, const char* plan) {
   const dim3 gd((unsigned)grid), bd(1u << NT);
   if constexpr (sizeof(R) == 4) {
     if (nrb == 4)
-      launch_reg<R, 4, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, plan);
+      launch_reg<R, 4, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
     else
-      launch_reg<R, 5, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, plan);
+      launch_reg<R, 5, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
   } else {
     if (nrb == 3)
-      launch_reg<R, 3, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, plan);
+      launch_reg<R, 3, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
     else
-      launch_reg<R, 4, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, plan);
+      launch_reg<R, 4, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
   }
 }
 
@@ -845,11 +859,19 @@ static int tile_pass_impl(const void* source, void* state, int nqubits, int L, c
       per_cu = std::min(per_cu, 2048 / bs);
       per_cu = std::max(per_cu, 1);
       const u64 rgrid = std::min<u64>(ntiles, (u64)cus * per_cu);
+      if (plan.size() <= sizeof(PlanArg)) {
+        PlanArg arg;
+        std::memcpy(arg.data, plan.data(), plan.size());
+        std::memset(arg.data + plan.size(), 0, sizeof(arg) - plan.size());
+        launch_tile_reg<R>(nrb, TB - nrb, rgrid, lds_reg, s, src, st, ntiles, tins, arg, nullptr);
+        return check_launch("apply_tile_pass launch");
+      }
       void* dplan = nullptr;
       int ticket = -1;
       int rc = ring_upload(plan.data(), plan.size(), s, &dplan, &ticket);
       if (rc) return rc;
-      launch_tile_reg<R>(nrb, TB - nrb, rgrid, lds_reg, s, src, st, ntiles, tins, static_cast<const char*>(dplan));
+      launch_tile_reg<R>(nrb, TB - nrb, rgrid, lds_reg, s, src, st, ntiles, tins, NoPlan{},
+                         static_cast<const char*>(dplan));
       rc = check_launch("apply_tile_pass launch");
       ring_release(ticket, s);
       return rc;
