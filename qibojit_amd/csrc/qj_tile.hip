@@ -691,14 +691,18 @@ static void device_limits(int* cus, size_t* max_lds) {
 
 // Register bits of the register kernel: 4 by default (QJ_TILE_NRB overrides:
 // 4/5 for complex64, 3/4 for complex128), at least the widest dense op.
-// Returns 0 when the pass needs the LDS kernel.
-static int tile_register_bits(bool dbl, int maxk) {
+// Register bits per thread; 0 when the pass needs the LDS kernel.  Four, or
+// what the widest dense op needs; complex128 takes three where each tile has a
+// CU to itself: eight waves a CU instead of four hide more of the re-layouts'
+// latency than the extra ones cost (random circuits of 16 to 20 qubits 2-6%
+// faster, QFTs and energies the same; with 16 tiles a CU, 14% slower).
+static int tile_register_bits(bool dbl, int maxk, u64 ntiles, int cus) {
   const char* kern = std::getenv("QJ_TILE_KERNEL");
   if (kern && std::strcmp(kern, "lds") == 0) return 0;
   const char* e = std::getenv("QJ_TILE_NRB");
   const int v = e ? std::atoi(e) : 0;
   const int lo = dbl ? 3 : 4, hi = dbl ? 4 : 5;
-  int nrb = (v >= lo && v <= hi) ? v : 4;
+  int nrb = (v >= lo && v <= hi) ? v : ntiles <= (u64)cus ? lo : 4;
   if (maxk > nrb) nrb = maxk;
   return nrb <= hi ? nrb : 0;
 }
@@ -814,7 +818,10 @@ static int tile_pass_impl(const void* source, void* state, int nqubits, int L, c
   cplx<R>* st = static_cast<cplx<R>*>(state);
   const char* cdata = static_cast<const char*>(data);
 
-  const int nrb = tile_register_bits(sizeof(R) == 8, maxk);
+  int cus = 0;
+  size_t max_lds = 0;
+  device_limits(&cus, &max_lds);
+  const int nrb = tile_register_bits(sizeof(R) == 8, maxk, ntiles, cus);
   if (nrb) {
     RegPlanIn in;
     std::memset(&in, 0, sizeof(in));
@@ -838,9 +845,6 @@ static int tile_pass_impl(const void* source, void* state, int nqubits, int L, c
     std::vector<char> plan;
     RegHead hh;
     size_t lds_reg = 0;
-    int cus = 0;
-    size_t max_lds = 0;
-    device_limits(&cus, &max_lds);
     const bool planned = reg_plan(in, plan);
     if (planned) {
       std::memcpy(&hh, plan.data(), sizeof(hh));
