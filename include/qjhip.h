@@ -202,6 +202,11 @@ int qj_apply_tile_pass(void* state, int dtype, int nqubits, int low_bits,
 int qj_apply_tile_pass_from(const void* source, void* state, int dtype, int nqubits, int low_bits,
                             const int32_t* high_bits, int nhigh, const qj_tile_op* ops, int nops, const void* data,
                             uint64_t data_bytes, void* stream);
+/* The same from `source` after bit swaps: bit b of the state is bit
+ * source_bits[b] of the source (nqubits entries, disjoint swaps; NULL: none). */
+int qj_apply_tile_pass_permuted(const void* source, const int32_t* source_bits, void* state, int dtype, int nqubits,
+                                int low_bits, const int32_t* high_bits, int nhigh, const qj_tile_op* ops, int nops,
+                                const void* data, uint64_t data_bytes, void* stream);
 
 /* ---- gate lists: planned into tile passes and run, one call per list ----
  * A record is {code, ntargets, ncontrols, targets..., controls...} (qubits,

@@ -45,6 +45,7 @@ SIGNATURES = {
     "qj_apply_two_qubit": [_vp, _i32, _i32, _i32, _i32, _i32, _pi32, _i32, _vp, _vp],
     "qj_apply_multi_qubit": [_vp, _i32, _i32, _pi32, _i32, _pi32, _i32, _vp, _vp],
     "qj_apply_tile_pass": [_vp, _i32, _i32, _i32, _pi32, _i32, _vp, _i32, _vp, _u64, _vp],
+    "qj_apply_tile_pass_permuted": [_vp, _pi32, _vp, _i32, _i32, _i32, _pi32, _i32, _vp, _i32, _vp, _u64, _vp],
     "qj_apply_tile_pass_from": [_vp, _vp, _i32, _i32, _i32, _pi32, _i32, _vp, _i32, _vp, _u64, _vp],
     "qj_run_gates": [_vp, _i32, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp, _i64, _pi32, _vp],
     "qj_apply_bit_swaps": [_vp, _i32, _i32, _pi32, _i32, _vp],

@@ -15,6 +15,14 @@
 // ladder becomes one op), and the ops are ordered so that as many dense
 // targets as possible share the kernel's register bits.
 //
+// A circuit that ends with swaps of many bits (a QFT) and starts from another
+// buffer has them moved to its front: SWAPs G = G' SWAPs with the bits of G
+// exchanged, and the first pass, which reads that buffer anyway, reads it
+// permuted (|0...0> is its own permutation).  The first tile then also holds
+// the bits that are lowest in the source, so that its loads are whole lines.
+// A 30-qubit complex64 QFT went from 19.5 to 17.1 ms, a 28-qubit complex128 one
+// from 9.3 to 7.65; with 12 to 20 qubits it takes as long or up to 12% less.
+//
 // The same steps in Python, cutting the list in order, took about 8 us a gate,
 // more than the device needed: 20 qubits, 600 gates 5.3 -> 1.07 ms (29 passes
 // instead of 43); the two-layer 26-qubit ansatz and its energy 5.9 -> 4.65 ms;
@@ -57,6 +65,7 @@ struct Run {
   hipStream_t stream;
   std::vector<c128> pool;
   std::vector<GateOp> ops;  // in circuit order
+  std::vector<int32_t> source_bits;  // state bit -> source bit, where swaps moved to the front
   int npasses = 0;
 };
 
@@ -336,9 +345,14 @@ int emit_tile(Run& run, std::vector<Item>& items, u64 high) {
     }
   }
   const int ga = (nout + 1) / 2, gb = nout - ga;
+  const bool permuted = run.from_source && !run.source_bits.empty();
   u64 lane_bits = 0;
-  for (int b = 0; b < run.nbits; ++b)
-    if (local[b] >= 0 && local[b] < 6) lane_bits |= bit(b);
+  for (int b = 0, lanes = 0; b < run.nbits && lanes < 6; ++b) {
+    const int sb = permuted ? run.source_bits[b] : b;  // the state bit that the source keeps at b
+    if (local[sb] < 0) continue;
+    lane_bits |= bit(sb);
+    ++lanes;
+  }
   order_items(items, lane_bits);
 
   std::vector<qj_tile_op> ops;
@@ -416,8 +430,9 @@ int emit_tile(Run& run, std::vector<Item>& items, u64 high) {
   }
   const void* src = run.from_source ? run.source : run.state;
   run.from_source = false;
-  return qj_apply_tile_pass_from(src, run.state, run.dtype, run.nbits, low, hb, tb - low, ops.data(), (int)ops.size(),
-                                 data.data(), data.size(), run.stream);
+  return qj_apply_tile_pass_permuted(src, permuted ? run.source_bits.data() : nullptr, run.state, run.dtype, run.nbits,
+                                     low, hb, tb - low, ops.data(), (int)ops.size(), data.data(), data.size(),
+                                     run.stream);
 }
 
 // The state itself before a pass that works in place.
@@ -427,7 +442,45 @@ int fill_state(Run& run) {
   if (run.plan_only) return QJ_OK;
   const u64 n = u64(1) << run.nbits;
   if (!run.source) return qj_initial_state(run.state, run.dtype, n, run.stream);
-  return qj_memcpy_dtod(run.state, run.source, n * elem_size(run.dtype), run.stream);
+  const int rc = qj_memcpy_dtod(run.state, run.source, n * elem_size(run.dtype), run.stream);
+  if (rc || run.source_bits.empty()) return rc;
+  std::vector<int32_t> pairs;
+  for (int b = 0; b < run.nbits; ++b)
+    if (b < run.source_bits[b]) {
+      pairs.push_back(b);
+      pairs.push_back(run.source_bits[b]);
+    }
+  return qj_apply_bit_swaps(run.state, run.dtype, run.nbits, pairs.data(), (int)pairs.size() / 2, run.stream);
+}
+
+// Moves swaps of many bits from the end of the circuit to its front (see the
+// top).  Returns the bits to keep in the first tile for its loads.
+u64 fold_swaps(Run& run, u64 low_mask) {
+  if (!run.from_source || run.nbits > 56) return 0;
+  u64 bits = 0;
+  size_t j = run.ops.size();
+  for (; j > 0 && run.ops[j - 1].kind == QJ_TILE_SWAP && !(run.ops[j - 1].X & bits); --j) bits |= run.ops[j - 1].X;
+  if (j == 0 || __builtin_popcountll(bits & ~low_mask) <= run.max_high) return 0;
+  std::vector<int32_t> to(run.nbits);
+  for (int b = 0; b < run.nbits; ++b) to[b] = b;
+  for (size_t i = j; i < run.ops.size(); ++i) std::swap(to[run.ops[i].tg[0]], to[run.ops[i].tg[1]]);
+  u64 keep = 0;  // whole 128-byte lines of the source
+  for (int b = 0; run.source && (elem_size(run.dtype) << b) < 128; ++b) keep |= bit(to[b]) & ~low_mask;
+  if (__builtin_popcountll(keep) >= run.max_high) return 0;
+  run.ops.resize(j);
+  for (GateOp& op : run.ops) {
+    if (op.kind == QJ_TILE_PHASE) {
+      if (op.tb >= 0) op.tb = to[op.tb];
+    } else {
+      for (int u = 0; u < op.k; ++u) op.tg[u] = to[op.tg[u]];
+    }
+    u64 ctrl = 0;
+    for (u64 m = op.ctrl; m; m &= m - 1) ctrl |= bit(to[__builtin_ctzll(m)]);
+    op.ctrl = ctrl;
+    set_masks(op);
+  }
+  if (run.source) run.source_bits = std::move(to);
+  return keep;
 }
 
 // The pending ops in order: those that earlier passes left behind, then the
@@ -460,6 +513,7 @@ int run_pending(Run& run) {
   const int esize = (int)elem_size(run.dtype);
   const u64 low_mask = bit(std::min(run.low, run.nbits)) - 1;
   const u64 all = bit(run.nbits) - 1;
+  u64 first_high = fold_swaps(run, low_mask);
   Pending pend{run.ops, {}, 0};
   std::vector<int> keep;
   std::vector<Item> items;
@@ -476,6 +530,7 @@ int run_pending(Run& run) {
         pairs.push_back(pend[j].tg[1]);
       }
       pend.consume(lead, keep);
+      first_high = 0;
       int rc = fill_state(run);
       ++run.npasses;
       if (!rc && !run.plan_only)
@@ -483,7 +538,7 @@ int run_pending(Run& run) {
       if (rc) return rc;
       continue;
     }
-    u64 high = 0, bx = 0, bz = 0;
+    u64 high = first_high, bx = 0, bz = 0;
     size_t bytes = 0, i = 0;
     while (i < pend.size() && bx != all) {  // with every bit changed by an op left behind, none commutes
       const size_t nrun = swap_run(pend, i, &bits);
@@ -513,6 +568,11 @@ int run_pending(Run& run) {
       if (take) high = need;
       i += n;
     }
+    if (items.empty() && first_high) {  // a wide gate comes first: without the load's bits
+      first_high = 0;
+      continue;
+    }
+    first_high = 0;
     if (items.empty()) return set_error(QJ_EVALUE, "run_gates: a gate does not fit a tile");
     pend.consume(i, keep);
     const int rc = run.dtype == QJ_COMPLEX64 ? emit_tile<float>(run, items, high) : emit_tile<double>(run, items, high);

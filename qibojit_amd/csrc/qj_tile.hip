@@ -55,9 +55,15 @@ constexpr int kTileLA = 8;  // tile bits indexing phase table A
 // their own, cost a pass of a 20-qubit circuit (24 gates, 31 us) 7 us.  The
 // 20-qubit random circuit of depth 20 went from 1.07 to 0.87 ms.
 struct PlanArg {
-  alignas(16) char data[3584];
+  alignas(16) char data[3520];
 };
 struct NoPlan {};
+// Where a permuted source (the last swaps of a circuit, moved to its front)
+// keeps the bits outside the tile; n = 0: where the state does.
+struct SourceBits {
+  int n;
+  u64 pos[7];  // eight positions a word
+};
 
 struct TileSpec {
   int L;                       // low contiguous bits
@@ -350,7 +356,8 @@ __device__ __forceinline__ u64 uni64(u64 v) {
 // parameter would be a per-thread copy), NoPlan when it is at plan_buf.
 template <typename R, int NRB, int BSMAX, int WPE, typename Plan>
 __global__ void __launch_bounds__(BSMAX, WPE)
-    k_tile_reg(Plan, const cplx<R>* src, cplx<R>* st, u64 ntiles, Ins tins, const char* __restrict__ plan_buf) {
+    k_tile_reg(Plan, const cplx<R>* src, cplx<R>* st, u64 ntiles, Ins tins, const char* __restrict__ plan_buf,
+               SourceBits sb) {
   constexpr int NR = 1 << NRB;
   const char* plan = plan_buf;
   if constexpr (std::is_same<Plan, PlanArg>::value) plan = (const char*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -417,9 +424,18 @@ __global__ void __launch_bounds__(BSMAX, WPE)
     if (tid < nphase) f[tid] = reg_phase_outside<R>(reinterpret_cast<const cplx<R>*>(plan + ftab[tid]), ga, t);
     cplx<R> x[NR];
     if (src) {  // uniform
+      u64 from = base;
+      if (sb.n) {
+        from = 0;
+        for (int j = 0; 8 * j < sb.n; ++j) {
+          const u64 w = sb.pos[j], tj = t >> (8 * j);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) from |= ((tj >> i) & 1) << ((w >> (8 * i)) & 63);
+        }
+      }
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
-        const char* p = reinterpret_cast<const char*>(src + (base | reg_state_offset<NRB>(ld_rb, r)));
+        const char* p = reinterpret_cast<const char*>(src + (from | reg_state_offset<NRB>(ld_rb, r)));
         x[r] = *reinterpret_cast<const cplx<R>*>(p + ld_thr_b);
       }
     } else {  // |0...0>
@@ -709,35 +725,39 @@ static int tile_register_bits(bool dbl, int maxk, u64 ntiles, int cus) {
 
 template <typename R, int NRB, int BSMAX, int WPE, typename Plan>
 static void launch_reg(dim3 gd, dim3 bd, size_t lds, hipStream_t s, const cplx<R>* src, cplx<R>* st, u64 ntiles,
-                       const Ins& tins, const Plan& arg, const char* plan) {
+                       const Ins& tins, const Plan& arg, const char* plan, const SourceBits& sb) {
   // dynamic LDS above 64 KiB needs the kernel's limit raised first
   if (lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tile_reg<R, NRB, BSMAX, WPE, Plan>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  k_tile_reg<R, NRB, BSMAX, WPE><<<gd, bd, lds, s>>>(arg, src, st, ntiles, tins, plan);
+  k_tile_reg<R, NRB, BSMAX, WPE><<<gd, bd, lds, s>>>(arg, src, st, ntiles, tins, plan, sb);
 }
 
 template <typename R, typename Plan>
 static void launch_tile_reg(int nrb, int NT, u64 grid, size_t lds, hipStream_t s, const cplx<R>* src, cplx<R>* st,
-                            u64 ntiles, const Ins& tins, const Plan& arg, const char* plan) {
+                            u64 ntiles, const Ins& tins, const Plan& arg, const char* plan, const SourceBits& sb) {
   const dim3 gd((unsigned)grid), bd(1u << NT);
   if constexpr (sizeof(R) == 4) {
     if (nrb == 4)
-      launch_reg<R, 4, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
+      launch_reg<R, 4, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan, sb);
     else
-      launch_reg<R, 5, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
+      launch_reg<R, 5, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan, sb);
   } else {
     if (nrb == 3)
-      launch_reg<R, 3, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
+      launch_reg<R, 3, 512, 4>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan, sb);
     else
-      launch_reg<R, 4, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan);
+      launch_reg<R, 4, 256, 2>(gd, bd, lds, s, src, st, ntiles, tins, arg, plan, sb);
   }
 }
 
 template <typename R>
-static int tile_pass_impl(const void* source, void* state, int nqubits, int L, const int32_t* high, int nhigh,
-                          const qj_tile_op* ops, int nops, const void* data, u64 data_bytes,
-                          hipStream_t s) {
+static int bit_swaps_impl(void* state, int nqubits, const int32_t* pairs, int npairs, hipStream_t s);
+
+// source_bits (or null): state bit -> bit of the source that holds it.
+template <typename R>
+static int tile_pass_impl(const void* source, const int32_t* source_bits, void* state, int nqubits, int L,
+                          const int32_t* high, int nhigh, const qj_tile_op* ops, int nops, const void* data,
+                          u64 data_bytes, hipStream_t s) {
   const int TB = L + nhigh;
   if (nqubits < 1 || nqubits > 62) return set_error(QJ_EVALUE, "apply_tile_pass: bad nqubits %d", nqubits);
   if (L < 1 || nhigh < 0 || nhigh > kTileMaxHighBits || TB > nqubits || TB > QJ_TILE_MAX_BITS)
@@ -842,6 +862,18 @@ static int tile_pass_impl(const void* source, void* state, int nqubits, int L, c
       return !(e && std::strcmp(e, "0") == 0);
     }();
     in.reg_offsets = offsets;
+    int spos[kRegMaxBits];
+    SourceBits sb;
+    std::memset(&sb, 0, sizeof(sb));
+    if (source_bits) {
+      for (int b = 0; b < TB; ++b) spos[b] = source_bits[tins.pos[b]];
+      in.spos = spos;
+      for (int b = 0; b < nqubits; ++b)
+        if (!(tile_mask & (u64(1) << b))) {
+          sb.pos[sb.n / 8] |= (u64)source_bits[b] << (8 * (sb.n % 8));
+          ++sb.n;
+        }
+    }
     std::vector<char> plan;
     RegHead hh;
     size_t lds_reg = 0;
@@ -867,7 +899,7 @@ static int tile_pass_impl(const void* source, void* state, int nqubits, int L, c
         PlanArg arg;
         std::memcpy(arg.data, plan.data(), plan.size());
         std::memset(arg.data + plan.size(), 0, sizeof(arg) - plan.size());
-        launch_tile_reg<R>(nrb, TB - nrb, rgrid, lds_reg, s, src, st, ntiles, tins, arg, nullptr);
+        launch_tile_reg<R>(nrb, TB - nrb, rgrid, lds_reg, s, src, st, ntiles, tins, arg, nullptr, sb);
         return check_launch("apply_tile_pass launch");
       }
       void* dplan = nullptr;
@@ -875,11 +907,25 @@ static int tile_pass_impl(const void* source, void* state, int nqubits, int L, c
       int rc = ring_upload(plan.data(), plan.size(), s, &dplan, &ticket);
       if (rc) return rc;
       launch_tile_reg<R>(nrb, TB - nrb, rgrid, lds_reg, s, src, st, ntiles, tins, NoPlan{},
-                         static_cast<const char*>(dplan));
+                         static_cast<const char*>(dplan), sb);
       rc = check_launch("apply_tile_pass launch");
       ring_release(ticket, s);
       return rc;
     }
+  }
+
+  // the LDS kernel reads its source as it is: permute first
+  if (source_bits) {
+    int rc = qj_memcpy_dtod(state, source, (u64(1) << nqubits) * sizeof(cplx<R>), s);
+    std::vector<int32_t> pairs;
+    for (int b = 0; b < nqubits; ++b)
+      if (b < source_bits[b]) {
+        pairs.push_back(b);
+        pairs.push_back(source_bits[b]);
+      }
+    if (!rc) rc = bit_swaps_impl<R>(state, nqubits, pairs.data(), (int)pairs.size() / 2, s);
+    if (rc) return rc;
+    src = st;
   }
 
   // LDS kernel: ops and data travel in one staging upload, ops first (64 B
@@ -1023,15 +1069,31 @@ extern "C" int qj_apply_tile_pass(void* state, int dtype, int nqubits, int low_b
 extern "C" int qj_apply_tile_pass_from(const void* source, void* state, int dtype, int nqubits, int low_bits,
                                        const int32_t* high_bits, int nhigh, const qj_tile_op* ops, int nops,
                                        const void* data, uint64_t data_bytes, void* stream) {
+  return qj_apply_tile_pass_permuted(source, nullptr, state, dtype, nqubits, low_bits, high_bits, nhigh, ops, nops,
+                                     data, data_bytes, stream);
+}
+
+extern "C" int qj_apply_tile_pass_permuted(const void* source, const int32_t* source_bits, void* state, int dtype,
+                                           int nqubits, int low_bits, const int32_t* high_bits, int nhigh,
+                                           const qj_tile_op* ops, int nops, const void* data, uint64_t data_bytes,
+                                           void* stream) {
+  if (!source || source == state) {
+    if (source_bits && source) return set_error(QJ_EVALUE, "apply_tile_pass: a permuted source is another buffer");
+    source_bits = nullptr;  // |0...0> is its own permutation
+  }
+  if (source_bits && nqubits > 56) return set_error(QJ_EVALUE, "apply_tile_pass: %d qubits", nqubits);
+  for (int b = 0; source_bits && b < nqubits; ++b)
+    if (source_bits[b] < 0 || source_bits[b] >= nqubits || source_bits[source_bits[b]] != b)
+      return set_error(QJ_EVALUE, "apply_tile_pass: source bits must be disjoint swaps");
   if (!state) return set_error(QJ_EVALUE, "apply_tile_pass: null state");
   if (nops < 0 || (nops > 0 && !ops)) return set_error(QJ_EVALUE, "apply_tile_pass: bad ops");
   if (nhigh > 0 && !high_bits) return set_error(QJ_EVALUE, "apply_tile_pass: null high bits");
   if (data_bytes > 0 && !data) return set_error(QJ_EVALUE, "apply_tile_pass: null data");
   hipStream_t s = (hipStream_t)stream;
   if (dtype == QJ_COMPLEX64)
-    return tile_pass_impl<float>(source, state, nqubits, low_bits, high_bits, nhigh, ops, nops, data, data_bytes, s);
+    return tile_pass_impl<float>(source, source_bits, state, nqubits, low_bits, high_bits, nhigh, ops, nops, data, data_bytes, s);
   if (dtype == QJ_COMPLEX128)
-    return tile_pass_impl<double>(source, state, nqubits, low_bits, high_bits, nhigh, ops, nops, data, data_bytes, s);
+    return tile_pass_impl<double>(source, source_bits, state, nqubits, low_bits, high_bits, nhigh, ops, nops, data, data_bytes, s);
   return set_error(QJ_EVALUE, "apply_tile_pass: dtype must be complex64/complex128");
 }
 

@@ -382,6 +382,7 @@ struct RegPlanIn {
   const char* data;
   u64 lds_cap;                 // largest LDS part a workgroup can hold
   bool reg_offsets = true;     // add the per-segment register offsets when they fit
+  const int* spos = nullptr;   // tile bit -> source bit, where the loads read a permuted source
 };
 
 inline int popc32(uint32_t v) { return __builtin_popcount(v); }
@@ -444,7 +445,12 @@ inline bool reg_plan(const RegPlanIn& in, std::vector<char>& blob) {
       if (((allowed >> b) & 1) && !((u >> b) & 1)) u |= uint32_t(1) << b;
     return u;
   };
-  const uint32_t ld_lanes = (uint32_t(1) << kRegLanes) - 1;
+  // load lanes: the tile bits lowest in what is loaded
+  std::vector<int> ld_order(TB);
+  for (int b = 0; b < TB; ++b) ld_order[b] = b;
+  if (in.spos) std::sort(ld_order.begin(), ld_order.end(), [&](int a, int b) { return in.spos[a] < in.spos[b]; });
+  uint32_t ld_lanes = 0;
+  for (int b = 0; b < kRegLanes; ++b) ld_lanes |= uint32_t(1) << ld_order[b];
   uint32_t st_lanes = 0;
   for (int b = 0; b < kRegLanes; ++b) st_lanes |= uint32_t(1) << phys[b];
   std::vector<uint32_t> regs;
@@ -480,7 +486,7 @@ inline bool reg_plan(const RegPlanIn& in, std::vector<char>& blob) {
     const uint32_t thr = all & ~regs[s];
     std::vector<int> lanes;
     if (s == 0) {
-      for (int b = 0; b < kRegLanes; ++b) lanes.push_back(b);
+      for (int b = 0; b < kRegLanes; ++b) lanes.push_back(ld_order[b]);
     } else if (s == nseg - 1) {
       for (int b = 0; b < kRegLanes; ++b) lanes.push_back(phys[b]);
     } else {
@@ -667,7 +673,7 @@ inline bool reg_plan(const RegPlanIn& in, std::vector<char>& blob) {
   h.had_scale = had_scale;
   h.nhad = nhad;
   for (int b = 0; b < TB; ++b) {
-    h.gbit_ld[b] = (uint8_t)in.gpos[b];
+    h.gbit_ld[b] = (uint8_t)(in.spos ? in.spos[b] : in.gpos[b]);
     h.gbit_st[b] = (uint8_t)in.gpos[inv[b]];
   }
 
