@@ -66,8 +66,9 @@ _CHANNEL_APPLY = getattr(getattr(gate_classes, "Channel", None), "apply_density_
 
 # Gates planned together by the fused executor.  The planner looks through all
 # of them for what a pass can take; the device waits for the first run's
-# records, about 2 us each.
-_RECORDS_PER_RUN = 512
+# records, about 1 us each.  A QFT of up to 44 qubits is one run, so that its
+# last swaps meet its initial state.
+_RECORDS_PER_RUN = 1024
 
 
 def _dtype_name(dtype):

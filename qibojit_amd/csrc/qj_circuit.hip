@@ -23,9 +23,14 @@
 // A 30-qubit complex64 QFT went from 19.5 to 17.1 ms, a 28-qubit complex128 one
 // from 9.3 to 7.65; with 12 to 20 qubits it takes as long or up to 12% less.
 //
+// A pass is closed when its plan would outgrow the kernel's LDS share, counted
+// item by item as the plan is laid out (what a merged phase adds, not what it
+// would take alone): with a rough budget of 12 of the 15 KiB a 32-qubit
+// complex128 QFT took one pass more (175 instead of 155 ms), and 20 qubits, 600
+// gates 0.82 instead of 0.68 ms.
+//
 // The same steps in Python, cutting the list in order, took about 8 us a gate,
-// more than the device needed: 20 qubits, 600 gates 5.3 -> 1.07 ms (29 passes
-// instead of 43); the two-layer 26-qubit ansatz and its energy 5.9 -> 4.65 ms;
+// more than the device needed: 20 qubits, 600 gates 5.3 -> 1.07 ms; the two-layer 26-qubit ansatz and its energy 5.9 -> 4.65 ms;
 // two layers of a noisy 12-qubit density matrix 1.83 -> 1.17 ms.
 #include <algorithm>
 #include <cmath>
@@ -34,6 +39,7 @@
 #include <vector>
 
 #include "qj_common.h"
+#include "qj_tile_reg.h"
 
 namespace qj {
 namespace {
@@ -218,14 +224,17 @@ int push_record(Run& run, int nqubits, bool density, const int32_t* rec, const d
 }
 
 // --------------------------------------------------------------- passes --
-// LDS bytes of an item in the register kernel's plan, and their budget: the
-// kernel keeps 15 KiB of plan next to a tile, segments included.
-constexpr size_t kPassBudget = 12 * 1024;
-size_t item_bytes(const GateOp& op, int esize) {
-  const size_t head = 56 + 16;
-  if (op.kind == QJ_TILE_SWAP) return 0;
-  if (op.kind == QJ_TILE_DENSE) return head + (size_t(1) << (2 * op.k)) * esize;
-  return head + (esize == 8 ? 88 : 84) * (size_t)esize;  // phase tables
+// LDS bytes of an item in the register kernel's plan (a dense op may also open
+// a segment), and their budget: what the plan may take next to a tile, less the
+// first and the last segment and three paddings.  A 32-qubit complex128 QFT needs
+// nearly all of it in its last pass.
+constexpr size_t kPassBudget = kRegPlanLds - 2 * sizeof(RegSeg) - 3 * 16;
+bool one_factor(const Item& it) { return it.th.empty() || (it.th.size() == 1 && it.op.c0 == 0.0); }
+size_t item_bytes(const Item& it, int esize) {
+  const size_t head = sizeof(RegOp) + sizeof(u64);
+  if (it.op.kind == QJ_TILE_SWAP) return 0;
+  if (it.op.kind == QJ_TILE_DENSE) return head + sizeof(RegSeg) + (size_t(1) << (2 * it.op.k)) * esize;
+  return head + (one_factor(it) ? 16 : (esize == 8 ? 100 : 84) * (size_t)esize);  // largest phase tables
 }
 
 bool symmetric(const Item& it) {
@@ -267,18 +276,34 @@ bool merge(Item& it, const Item& p) {
 }
 
 // Appends an op to a pass: phases join the latest item they can merge with
-// while everything after it commutes with them.
-void add_item(std::vector<Item>& items, const GateOp& op) {
+// while everything after it commutes with them.  False, and nothing is
+// changed, if the pass's plan would grow over its budget.
+bool add_item(std::vector<Item>& items, const GateOp& op, int esize, size_t* bytes) {
   Item it;
   it.op = op;
   if (op.kind == QJ_TILE_PHASE) {
     if (op.tb >= 0) it.th.push_back({op.tb, op.th});
     for (size_t j = items.size(), tries = 0; j-- > 0 && tries < 64; ++tries) {
-      if (items[j].op.kind == QJ_TILE_PHASE && merge(items[j], it)) return;
+      if (items[j].op.kind == QJ_TILE_PHASE) {
+        Item old = items[j];
+        if (merge(items[j], it)) {
+          const size_t now = *bytes - item_bytes(old, esize) + item_bytes(items[j], esize);
+          if (now > kPassBudget && now > *bytes) {
+            items[j] = std::move(old);
+            return false;
+          }
+          *bytes = now;
+          return true;
+        }
+      }
       if (items[j].op.X & op.Z) break;
     }
   }
+  const size_t more = item_bytes(it, esize);
+  if (!items.empty() && more && *bytes + more > kPassBudget) return false;
+  *bytes += more;
   items.push_back(std::move(it));
+  return true;
 }
 
 // Orders the items so that runs of dense ops share the kernel's four
@@ -385,7 +410,7 @@ int emit_tile(Run& run, std::vector<Item>& items, u64 high) {
       o.offset = room(n * sizeof(cplx<R>));
       cplx<R>* m = reinterpret_cast<cplx<R>*>(data.data() + o.offset);
       for (size_t j = 0; j < n; ++j) put(m + j, run.pool[it.op.mat + j]);
-    } else if (it.th.empty() || (it.th.size() == 1 && it.op.c0 == 0.0)) {
+    } else if (one_factor(it)) {
       // one factor where every bit is 1
       o.kind = QJ_TILE_SCALE;
       if (!it.th.empty()) ctrl |= bit(it.th[0].first);
@@ -545,25 +570,19 @@ int run_pending(Run& run) {
       const size_t n = nrun >= 2 ? nrun : 1;  // swaps of a run stay together
       bool take = true;
       u64 need = high;
-      size_t more = 0;
       for (size_t j = i; j < i + n; ++j) {
         const GateOp& op = pend[j];
         take = take && !((op.X | op.Z) & bx) && !(op.X & bz);
         need |= op.X & ~low_mask;
-        more += item_bytes(op, esize);
       }
-      take = take && __builtin_popcountll(need) <= run.max_high && (items.empty() || bytes + more <= kPassBudget);
+      take = take && __builtin_popcountll(need) <= run.max_high;
       for (size_t j = i; j < i + n; ++j) {
         const GateOp& op = pend[j];
-        if (!take) {
-          bx |= op.X;
-          bz |= op.Z;
-          keep.push_back(pend.id(j));
-          continue;
-        }
-        const size_t count = items.size();
-        add_item(items, op);
-        if (items.size() > count) bytes += item_bytes(op, esize);  // merged phases take no room
+        take = take && add_item(items, op, esize, &bytes);  // swaps take no room: a run is not cut
+        if (take) continue;
+        bx |= op.X;
+        bz |= op.Z;
+        keep.push_back(pend.id(j));
       }
       if (take) high = need;
       i += n;

@@ -683,10 +683,8 @@ static void lds_kernel_data(const qj_tile_op* ops, int nops, const char* data, i
   }
 }
 
-// LDS of one CU, and the share of it a register-kernel plan may take next to
-// a 64 KiB tile (two workgroups per CU).
+// LDS of one CU.
 constexpr size_t kLdsPerCu = 160 * 1024;
-constexpr u64 kRegPlanLds = 15 * 1024;
 
 // Compute units and the largest LDS allocation of one workgroup, per device.
 static void device_limits(int* cus, size_t* max_lds) {

@@ -57,6 +57,9 @@ struct RegHead {
   uint8_t gbit_st[kRegMaxBits];  // physical tile bit -> state bit (store)
 };
 
+// Largest LDS part of a plan next to a 64 KiB tile (two workgroups per CU).
+constexpr u64 kRegPlanLds = 15 * 1024;
+
 struct RegSeg {
   int32_t o0, o1;                // ops [o0, o1) run in this layout
   int8_t slot[kRegMaxBits];      // slot -> physical tile bit
