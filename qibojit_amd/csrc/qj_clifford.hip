@@ -1439,7 +1439,6 @@ bool rows_plan(int n, int S, RowsPlan* p) {
   p->R = 1;
   if (nw <= 8)
     while (p->R < nw) p->R *= 2;
-  else if (const char* e = std::getenv("QJ_RT")) p->R = std::atoi(e);
   p->G = (nw + p->R - 1) / p->R;
   const int64_t C = 2 * (int64_t)n + S;
   p->dw = (int)(2 * ((C + 63) / 64));
@@ -1454,7 +1453,8 @@ const void* rows_kernel(int R) {
     case 1: return reinterpret_cast<const void*>(&k_cliff_measure_rows<1, SYM>);
     case 2: return reinterpret_cast<const void*>(&k_cliff_measure_rows<2, SYM>);
     case 4: return reinterpret_cast<const void*>(&k_cliff_measure_rows<4, SYM>);
-    default: return reinterpret_cast<const void*>(&k_cliff_measure_rows<8, SYM>);
+    case 8: return reinterpret_cast<const void*>(&k_cliff_measure_rows<8, SYM>);
+    default: return nullptr;
   }
 }
 
@@ -1464,6 +1464,8 @@ template <bool SYM>
 int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStream_t s, int* rc) {
   RowsPlan p;
   if (!rows_plan(a.n, a.S, &p)) return 0;
+  const void* kern = rows_kernel<SYM>(p.R);
+  if (!kern) return 0;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
@@ -1490,7 +1492,6 @@ int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStr
   *rc = ring_upload(qubits, (size_t)a.m * sizeof(int32_t), s, &dq, &ticket);
   if (*rc) return 1;
   a.qubits = static_cast<const int32_t*>(dq);
-  const void* kern = rows_kernel<SYM>(p.R);
   if (p.lds > 65536) (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
   void* args[] = {&a};
   if (p.G == 1) {

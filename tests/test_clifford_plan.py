@@ -1,0 +1,25 @@
+"""Shape of the one-launch Clifford measurement loop: host arithmetic."""
+
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SCRIPT = """
+from qibojit_amd import _native
+print([_native.lib().qj_clifford_forms_supported(n, m) for n in (1, 100, 256, 257, 1000, 4000) for m in (1, 100, 1000)])
+"""
+
+
+@pytest.mark.parametrize("value", ["0", "3", "8", "x"])
+def test_shape_depends_on_the_tableau_alone(value):
+    out = []
+    for env in ({}, {"QJ_RT": value}):
+        proc = subprocess.run([sys.executable, "-c", SCRIPT], cwd=ROOT, env={**os.environ, **env},
+                              capture_output=True, text=True, timeout=300)
+        assert proc.returncode == 0, proc.stderr[-500:]
+        out.append(proc.stdout)
+    assert out[0] == out[1]
