@@ -28,8 +28,6 @@
 // workgroup; 6.8 before), 4.4 at 1000 (32 workgroups; 26), 7.3 at 4000.  Two or
 // four words of rows per workgroup (fewer, larger) measured 8% and 40% slower
 // at 1000 qubits.
-constexpr int kRowsThreads = 512;
-constexpr int kRowsWaves = kRowsThreads / 64;
 constexpr int kRowsMaxSpins = 1 << 22;
 
 typedef unsigned long long post_t;
@@ -130,11 +128,7 @@ struct RowsArgs {
 template <int R, bool SYM>
 __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a) {
   extern __shared__ uint32_t rows_lds[];
-  __shared__ uint4 s_cnt[kRowsWaves * R];
-  __shared__ int s_best, s_ok, s_fetched;
-  __shared__ uint32_t s_par;
-  __shared__ int s_q[kRowsThreads];         // the next steps' qubits
-  __shared__ uint8_t s_draw[kRowsThreads];  // and random bits
+  __shared__ RowsShared<R, SYM> sh;
   const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
   const int g = (int)blockIdx.x, G = (int)gridDim.x;
   const int n = a.n, C = 2 * n + a.S, w0 = g * R, nw = (n + 31) >> 5;
@@ -164,18 +158,18 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
   int count = 0;
   bool det_any = false, ok = true;
   uint32_t scr_sign = 0;
-  int drawn = 0;  // random outcomes before s_draw[0]
+  int drawn = 0;  // random outcomes before sh.draw[0]
   lds_barrier();
   for (int i = 0; i < a.m; ++i) {
     const uint32_t tag = (uint32_t)i + 1;
     if ((i & (kRowsThreads - 1)) == 0) {  // uniform; the barrier above closed the last reads
-      s_q[t] = i + t < a.m ? a.qubits[i + t] : 0;
-      if (!SYM) s_draw[t] = count + t < a.m ? a.draws[count + t] : 0;
+      sh.q[t] = i + t < a.m ? a.qubits[i + t] : 0;
+      if (!SYM) sh.draw[t] = count + t < a.m ? a.draws[count + t] : 0;
       drawn = count;
       lds_barrier();
     }
-    const int q = s_q[i & (kRowsThreads - 1)];
-    const uint32_t draw = SYM ? 0u : (s_draw[count - drawn] & 1u);
+    const int q = sh.q[i & (kRowsThreads - 1)];
+    const uint32_t draw = SYM ? 0u : (sh.draw[count - drawn] & 1u);
     uint32_t hD[R], hS[R];
     int cand = -1;
     uint32_t par = 0;
@@ -235,10 +229,10 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
         }
         const bool all = __all(got);
         if (lane == 0) {
-          s_best = best;
-          s_par = px;
-          s_ok = all;
-          s_fetched = 1;
+          sh.best = best;
+          sh.par = px;
+          sh.ok = all;
+          sh.fetched = 1;
         }
       }
     }
@@ -246,9 +240,9 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
     int best = cand >= 0 ? cand : 0x7fffffff;
     uint32_t parity = par;
     if (G > 1) {
-      best = s_best;
-      parity = s_par;
-      ok = s_ok;
+      best = sh.best;
+      parity = sh.par;
+      ok = sh.ok;
       if (!ok) break;  // uniform
     }
     if (best != 0x7fffffff) {
@@ -262,9 +256,9 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
           got = got && await_word(data + (size_t)owner * a.dw + w, tag, &v);
           rowp[w] = v;
         }
-        if (!got) s_fetched = 0;
+        if (!got) sh.fetched = 0;
         lds_barrier();
-        ok = s_fetched;
+        ok = sh.fetched;
         if (!ok) break;  // uniform
       }
       const int r = t % R;
@@ -305,12 +299,12 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
       }
       count_lanes<R, 64>(d0, d1);
       count_lanes<R, 64>(s0, s1);
-      if (lane < R) s_cnt[wave * R + lane] = make_uint4(d0, d1, s0, s1);
+      if (lane < R) sh.cnt[wave * R + lane] = make_uint4(d0, d1, s0, s1);
       lds_barrier();
       ++count;
       {
         // every wave adds the waves' counters: lane l those of rows l % R
-        const uint4 v = s_cnt[lane % (kRowsWaves * R)];
+        const uint4 v = sh.cnt[lane % (kRowsWaves * R)];
         d0 = v.x;
         d1 = v.y;
         s0 = v.z;
@@ -353,7 +347,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
           for (int j = 0; j < 32 && 32 * w + j < a.S; ++j)
             a.forms[(size_t)i * (a.m + 1) + 32 * w + j] = (uint8_t)((sum >> j) & 1u);
         }
-        if (!got) s_fetched = 0;
+        if (!got) sh.fetched = 0;
       }
     } else {
       det_any = true;
@@ -369,9 +363,9 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
       }
       if (g == 0 && t == 0) a.sample[i] = (int32_t)parity;
     }
-    lds_barrier();  // the step's words, counters and s_* are read before the next writes
+    lds_barrier();  // the step's words, counters and sh are read before the next writes
     if (SYM && G > 1 && g == 0) {
-      ok = s_fetched;
+      ok = sh.fetched;
       lds_barrier();  // read before the next step sets it
       if (!ok) break;   // uniform
     }

@@ -21,6 +21,7 @@
 #include <cstring>
 #include <vector>
 
+#include "qj_cliff_plan.h"
 #include "qj_common.h"
 
 namespace qj {
@@ -1424,27 +1425,12 @@ void launch_circuit(uint32_t* tab, int nqubits, const uint32_t* ddesc, int64_t n
   }
 }
 
-// Shape of k_cliff_measure_rows for n qubits and S sign columns: one workgroup
-// up to 256 qubits (no exchange), else 32 rows each, so that every workgroup
-// is resident and its slice fits LDS.
-struct RowsPlan {
-  int R, G, dw;
-  size_t lds;
-};
+template <bool SYM>
 bool rows_plan(int n, int S, RowsPlan* p) {
-  const int nw = (n + 31) / 32;
   int cus = 0;
   size_t max_lds = 0;
   device_lds(&cus, &max_lds);
-  p->R = 1;
-  if (nw <= 8)
-    while (p->R < nw) p->R *= 2;
-  p->G = (nw + p->R - 1) / p->R;
-  const int64_t C = 2 * (int64_t)n + S;
-  p->dw = (int)(2 * ((C + 63) / 64));
-  p->lds = ((size_t)2 * C * p->R + 2 * (size_t)p->dw) * sizeof(uint32_t);
-  const size_t cap = std::min(kCliffLdsPerCu, std::max<size_t>(max_lds, 65536)) - 2048;  // static part
-  return p->G <= cus && p->G <= 256 && p->lds <= cap;
+  return rows_shape<SYM>(n, S, cus, std::min(kCliffLdsPerCu, std::max<size_t>(max_lds, 65536)), p);
 }
 
 template <bool SYM>
@@ -1463,7 +1449,7 @@ const void* rows_kernel(int R) {
 template <bool SYM>
 int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStream_t s, int* rc) {
   RowsPlan p;
-  if (!rows_plan(a.n, a.S, &p)) return 0;
+  if (!rows_plan<SYM>(a.n, a.S, &p)) return 0;
   const void* kern = rows_kernel<SYM>(p.R);
   if (!kern) return 0;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -1817,7 +1803,7 @@ int qj_clifford_rowsum(uint32_t* tab, int nqubits, const int64_t* h, const int64
 
 int qj_clifford_forms_supported(int nqubits, int m) {
   RowsPlan p;
-  return nqubits >= 1 && nqubits <= kCliffMaxQubits && m >= 1 && rows_plan(nqubits, m + 1, &p) ? 1 : 0;
+  return nqubits >= 1 && nqubits <= kCliffMaxQubits && m >= 1 && rows_plan<true>(nqubits, m + 1, &p) ? 1 : 0;
 }
 
 int qj_clifford_measurement_forms(const uint32_t* tab, int nqubits, const int32_t* qubits, int m, uint8_t* forms,
