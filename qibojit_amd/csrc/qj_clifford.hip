@@ -1460,24 +1460,38 @@ int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStr
   const int64_t W = cliff_words(a.n), C = 2 * (int64_t)a.n + 1;
   const size_t posts = (size_t)2 * p.G * (1 + p.dw);
   const size_t stage = SYM ? 0 : (size_t)2 * C * p.G * p.R, scratch = SYM ? 0 : (size_t)p.G * (p.dw + 1);
-  DeviceScratch* sc = nullptr;
-  *rc = scratch_for_current_device(&sc);
+  // Work space behind the qubit list in its ring slot, which the slot's event
+  // guards on every stream (up to about 700 qubits; always in the symbolic form
+  // with a few thousand sign columns), else the device's scratch, as the
+  // per-qubit kernels take it.
+  const size_t work = posts * sizeof(post_t) + (stage + scratch + 4) * sizeof(uint32_t);
+  const size_t list = ((size_t)a.m * sizeof(int32_t) + 15) & ~size_t(15);
+  const bool in_slot = list + work <= kRingSlotBytes;
+  void* dq = nullptr;
+  int ticket = -1;
+  *rc = ring_upload(qubits, (size_t)a.m * sizeof(int32_t), s, &dq, &ticket,
+                    in_slot ? list - (size_t)a.m * sizeof(int32_t) + work : 0);
   if (*rc) return 1;
-  *rc = scratch_reserve_big(sc, posts * sizeof(post_t) + (stage + scratch + 4) * sizeof(uint32_t), s);
-  if (*rc) return 1;
+  a.qubits = static_cast<const int32_t*>(dq);
+  void* area = static_cast<char*>(dq) + list;
+  if (!in_slot) {
+    DeviceScratch* sc = nullptr;
+    *rc = scratch_for_current_device(&sc);
+    if (!*rc) *rc = scratch_reserve_big(sc, work, s);
+    if (*rc) {
+      ring_release(ticket, s);
+      return 1;
+    }
+    area = sc->big;
+  }
   a.tab = tab;
   a.ws = cliff_stride(a.n);
   a.dw = p.dw;
-  a.hdr = static_cast<post_t*>(sc->big);
+  a.hdr = static_cast<post_t*>(area);
   a.data = a.hdr + (size_t)2 * p.G;
   a.stage = reinterpret_cast<uint32_t*>(a.hdr + posts);
   a.scratch = a.stage + stage;
   a.det_any = reinterpret_cast<int32_t*>(a.scratch + scratch);
-  void* dq = nullptr;
-  int ticket = -1;
-  *rc = ring_upload(qubits, (size_t)a.m * sizeof(int32_t), s, &dq, &ticket);
-  if (*rc) return 1;
-  a.qubits = static_cast<const int32_t*>(dq);
   if (p.lds > 65536) (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
   void* args[] = {&a};
   if (p.G == 1) {

@@ -111,9 +111,12 @@ int scratch_for_current_device(DeviceScratch** out);
 int scratch_reserve_big(DeviceScratch* sc, size_t bytes, hipStream_t stream);
 // Matrix staging: copies `bytes` from host `src` into a device slot ordered on
 // `stream`; returns the device pointer and a ticket to pass to ring_release
-// after the consuming kernel has been enqueued.
+// after the consuming kernel has been enqueued.  `room` more bytes of the slot,
+// behind the copy, are the caller's until then: work space that no other stream
+// or thread can hold.
+constexpr size_t kRingSlotBytes = 256 * 1024;  // a 7-qubit complex128 matrix
 int ring_upload(const void* src, size_t bytes, hipStream_t stream, void** dev,
-                int* ticket);
+                int* ticket, size_t room = 0);
 void ring_release(int ticket, hipStream_t stream);
 
 inline bool is_complex(int dtype) {

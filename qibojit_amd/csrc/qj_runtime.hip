@@ -76,7 +76,6 @@ int scratch_reserve_big(DeviceScratch* sc, size_t bytes, hipStream_t stream) {
 // recorded behind its consuming kernel has completed, so uploads never need a
 // per-gate host synchronisation.
 static constexpr int kSlots = 64;
-static constexpr size_t kSlotBytes = 256 * 1024;  // a 7-qubit complex128 matrix
 
 struct Ring {
   char* host = nullptr;
@@ -93,10 +92,10 @@ static Ring* g_ring[kMaxDevices] = {nullptr};
 static int ring_for_device(int dev, Ring** out) {
   if (!g_ring[dev]) {
     Ring* r = new Ring();
-    int rc = hip_status(hipHostMalloc((void**)&r->host, kSlots * kSlotBytes, hipHostMallocDefault),
+    int rc = hip_status(hipHostMalloc((void**)&r->host, kSlots * kRingSlotBytes, hipHostMallocDefault),
                         "pinned staging ring");
     if (rc) { delete r; return rc; }
-    rc = hip_status(hipMalloc((void**)&r->dev, kSlots * kSlotBytes), "device staging ring");
+    rc = hip_status(hipMalloc((void**)&r->dev, kSlots * kRingSlotBytes), "device staging ring");
     if (rc) { hipHostFree(r->host); delete r; return rc; }
     for (int i = 0; i < kSlots; ++i) {
       rc = hip_status(hipEventCreateWithFlags(&r->ev[i], hipEventDisableTiming), "ring event");
@@ -112,7 +111,7 @@ static int ring_for_device(int dev, Ring** out) {
 }
 
 int ring_upload(const void* src, size_t bytes, hipStream_t stream, void** dev_out,
-                int* ticket) {
+                int* ticket, size_t room) {
   int dev = 0;
   int rc = hip_status(hipGetDevice(&dev), "hipGetDevice");
   if (rc) return rc;
@@ -131,13 +130,13 @@ int ring_upload(const void* src, size_t bytes, hipStream_t stream, void** dev_ou
   }
   char* hsrc;
   char* ddst;
-  if (bytes <= kSlotBytes) {
-    hsrc = r->host + slot * kSlotBytes;
-    ddst = r->dev + slot * kSlotBytes;
+  if (bytes + room <= kRingSlotBytes) {
+    hsrc = r->host + slot * kRingSlotBytes;
+    ddst = r->dev + slot * kRingSlotBytes;
   } else {
     rc = hip_status(hipHostMalloc((void**)&hsrc, bytes, hipHostMallocDefault), "pinned matrix buffer");
     if (rc) return rc;
-    rc = hip_status(hipMalloc((void**)&ddst, bytes), "device matrix buffer");
+    rc = hip_status(hipMalloc((void**)&ddst, bytes + room), "device matrix buffer");
     if (rc) { hipHostFree(hsrc); return rc; }
     r->big_host[slot] = hsrc;
     r->big_dev[slot] = ddst;
