@@ -198,6 +198,9 @@ int push_record(Run& run, int nqubits, bool density, const int32_t* rec, const d
     op.kind = QJ_TILE_PHASE;
     op.tb = op.tg[0];
   } else {
+    // no rotation by an infinite angle; NaN runs through
+    if ((code == QJ_GATE_RX || code == QJ_GATE_RY || code == QJ_GATE_U3) && std::isinf(p[0]))
+      return set_error(QJ_EVALUE, "run_gates: rotation angle is infinite");
     c128 m[4];
     one_qubit_matrix(code, p, m);
     op.kind = QJ_TILE_DENSE;
