@@ -829,12 +829,14 @@ class HipBackend(Backend):
         return not (name in ("M", "Align", "CallbackGate") or "Channel" in name or hasattr(gate, "coefficients"))
 
     def _is_plain_state(self, state):
-        """A device tensor whose memory a kernel can read as the state."""
+        """A device tensor whose memory a kernel can read as the state (some
+        load 16 bytes at a time, so a view may have to be copied)."""
         return (
             isinstance(state, torch.Tensor)
             and state.device == self._torch_device
             and state.dtype in (torch.complex64, torch.complex128)
             and state.is_contiguous()
+            and state.data_ptr() % 16 == 0
             and not state.is_conj()
             and not state.is_neg()
         )
