@@ -309,16 +309,18 @@ bool add_item(std::vector<Item>& items, const GateOp& op, int esize, size_t* byt
   return true;
 }
 
-// Orders the items so that runs of dense ops share the kernel's four
-// register bits (each new register set re-lays the tile out through LDS);
+// Orders the items so that runs of dense ops share the kernel's register
+// bits (each new register set re-lays the tile out through LDS);
 // the first run avoids the six lowest tile bits, which the loads keep on
 // the lanes of a wave.
-void order_items(std::vector<Item>& items, u64 lane_bits) {
-  int nrb = 4;
+void order_items(std::vector<Item>& items, u64 lane_bits, int dtype, u64 ntiles) {
+  int maxk = 0;
   for (const Item& it : items) {
     if (it.op.kind == QJ_TILE_SWAP) return;  // swaps relabel bits on the way
-    if (it.op.kind == QJ_TILE_DENSE) nrb = std::max(nrb, it.op.k);
+    if (it.op.kind == QJ_TILE_DENSE) maxk = std::max(maxk, it.op.k);
   }
+  const int nrb = tile_register_bits(dtype, maxk, ntiles);
+  if (!nrb) return;  // the LDS kernel keeps no bits in registers
   std::vector<Item> out;
   out.reserve(items.size());
   std::vector<char> done(items.size(), 0);
@@ -381,7 +383,7 @@ int emit_tile(Run& run, std::vector<Item>& items, u64 high) {
     lane_bits |= bit(sb);
     ++lanes;
   }
-  order_items(items, lane_bits);
+  order_items(items, lane_bits, run.dtype, u64(1) << nout);
 
   std::vector<qj_tile_op> ops;
   std::vector<char> data;

@@ -703,16 +703,13 @@ static void device_limits(int* cus, size_t* max_lds) {
   *max_lds = dev >= 0 ? (size_t)mlds[dev] : 65536;
 }
 
-// Register bits of the register kernel: 4 by default (QJ_TILE_NRB overrides:
-// 4/5 for complex64, 3/4 for complex128), at least the widest dense op.
-// Register bits per thread; 0 when the pass needs the LDS kernel.  Four, or
-// what the widest dense op needs; complex128 takes three where each tile has a
-// CU to itself: eight waves a CU instead of four hide more of the re-layouts'
-// latency than the extra ones cost (random circuits of 16 to 20 qubits 2-6%
-// faster, QFTs and energies the same; with 16 tiles a CU, 14% slower).
-static int tile_register_bits(bool dbl, int maxk, u64 ntiles, int cus) {
+int tile_register_bits(int dtype, int maxk, u64 ntiles) {
+  const bool dbl = dtype == QJ_COMPLEX128;
   const char* kern = std::getenv("QJ_TILE_KERNEL");
   if (kern && std::strcmp(kern, "lds") == 0) return 0;
+  int cus = 0;
+  size_t max_lds = 0;
+  device_limits(&cus, &max_lds);
   const char* e = std::getenv("QJ_TILE_NRB");
   const int v = e ? std::atoi(e) : 0;
   const int lo = dbl ? 3 : 4, hi = dbl ? 4 : 5;
@@ -839,7 +836,7 @@ static int tile_pass_impl(const void* source, const int32_t* source_bits, void* 
   int cus = 0;
   size_t max_lds = 0;
   device_limits(&cus, &max_lds);
-  const int nrb = tile_register_bits(sizeof(R) == 8, maxk, ntiles, cus);
+  const int nrb = tile_register_bits(sizeof(R) == 8 ? QJ_COMPLEX128 : QJ_COMPLEX64, maxk, ntiles);
   if (nrb) {
     RegPlanIn in;
     std::memset(&in, 0, sizeof(in));

@@ -33,6 +33,19 @@
 
 namespace qj {
 
+// Register bits per thread of a pass of `ntiles` tiles whose widest dense op has
+// maxk targets; 0 when it needs the LDS kernel.  The planner orders the ops of a
+// pass by the same count.  Four, or what the widest dense op needs; complex128
+// takes three where each tile has a CU to itself: eight waves a CU instead of
+// four hide more of the re-layouts' latency than the extra ones cost.  12 to 20
+// qubits, 600 gates, three against four: one-target gates 10-11% faster, with
+// CNOTs 6-8%, a mixture with fSim 10-15%, QFTs 2-18%.  With 2 to 32 tiles a CU
+// lists of one-target gates are still 2-6% faster, but a noisy 12-qubit density
+// matrix (16 tiles a CU) takes 6% longer, the 26-qubit ansatz 2.5% and QFTs of 24
+// qubits or more 3%.  QJ_TILE_NRB overrides (4 or 5 for complex64, 3 or 4 for
+// complex128).
+int tile_register_bits(int dtype, int maxk, u64 ntiles);
+
 constexpr int kRegMaxSeg = 64;
 constexpr int kRegMaxBits = 16;
 constexpr int kRegLanes = 6;  // tile bits on the lanes of one wave

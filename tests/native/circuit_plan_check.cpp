@@ -19,9 +19,42 @@ int set_error(int code, const char* fmt, ...) {
   printf("\n");
   return code;
 }
+// The rule of the launch (qj_tile.hip) on 256 CUs.
+int tile_register_bits(int dtype, int maxk, u64 ntiles) {
+  const int most = dtype == QJ_COMPLEX128 ? 4 : 5;
+  const int bits = std::max(maxk, dtype == QJ_COMPLEX128 && ntiles <= 256 ? 3 : 4);
+  return bits <= most ? bits : 0;
+}
 }  // namespace qj
 
-static int g_permuted = 0;
+static int g_permuted = 0, g_segments = 0;
+
+// Register layouts of the pass's plan (0 where the LDS kernel runs it).
+static int segments(int dtype, int nq, int low, const int32_t* high, int nhigh, const int32_t* source_bits,
+                    const qj_tile_op* ops, int nops, const char* data) {
+  int maxk = 0, spos[kRegMaxBits];
+  for (int o = 0; o < nops; ++o)
+    if (ops[o].kind == QJ_TILE_DENSE) maxk = std::max(maxk, ops[o].k);
+  RegPlanIn in;
+  std::memset(&in, 0, sizeof(in));
+  in.TB = low + nhigh;
+  in.NRB = tile_register_bits(dtype, maxk, u64(1) << (nq - in.TB));
+  if (!in.NRB) return 0;
+  in.S = dtype == QJ_COMPLEX64 ? 5 : 4;
+  in.esize = (int)elem_size(dtype);
+  const int nout = nq - in.TB;
+  in.ga = (nout + 1) / 2;
+  in.gb = nout - in.ga;
+  for (int b = 0; b < in.TB; ++b) in.gpos[b] = b < low ? b : high[b - low];
+  for (int b = 0; source_bits && b < in.TB; ++b) spos[b] = source_bits[in.gpos[b]];
+  in.spos = source_bits ? spos : nullptr;
+  in.ops = ops;
+  in.nops = nops;
+  in.data = data;
+  in.lds_cap = kRegPlanLds;
+  std::vector<char> plan;
+  return reg_plan(in, plan) ? reinterpret_cast<const RegHead*>(plan.data())->nseg : 0;
+}
 
 template <typename R>
 static int host_pass(const void* source, const int32_t* source_bits, void* state, int nq, int low, const int32_t* high,
@@ -112,6 +145,7 @@ extern "C" int qj_apply_tile_pass_permuted(const void* source, const int32_t* so
                                            const qj_tile_op* ops, int nops, const void* data, uint64_t, void*) {
   g_permuted += source_bits != nullptr;
   const char* d = static_cast<const char*>(data);
+  g_segments = std::max(g_segments, segments(dtype, nqubits, low_bits, high_bits, nhigh, source_bits, ops, nops, d));
   return dtype == QJ_COMPLEX64
              ? host_pass<float>(source, source_bits, state, nqubits, low_bits, high_bits, nhigh, ops, nops, d)
              : host_pass<double>(source, source_bits, state, nqubits, low_bits, high_bits, nhigh, ops, nops, d);
@@ -299,6 +333,27 @@ static int check(std::mt19937_64& rng, int nq, bool density, int low, int max_hi
   return pass ? 0 : 1;
 }
 
+// Layers of one-target dense gates: the runs of a pass share register sets, so
+// its 12 or 13 bits take one set per 3 or 4 of them and at most two more (the
+// loads and the stores keep six bits on a wave's lanes).
+static int layers(int nq, int dtype, int low, int per_set) {
+  std::vector<int32_t> recs;
+  std::vector<double> params;
+  for (int g = 0; g < 10 * nq; ++g) {
+    recs.insert(recs.end(), {g % 3 ? QJ_GATE_RX : QJ_GATE_U3, 1, 0, g % nq});
+    params.insert(params.end(), g % 3 ? 1 : 3, 0.1 * g);
+  }
+  std::vector<double> st(size_t(2) << nq);
+  g_segments = 0;
+  const int rc = qj_run_gates(nullptr, 1, st.data(), dtype, nq, 0, low, 7, recs.data(), (int64_t)recs.size(),
+                              params.data(), (int64_t)params.size(), nullptr, nullptr);
+  const int limit = (low + 7 + per_set - 1) / per_set + 2;
+  const bool pass = rc == 0 && g_segments > 0 && g_segments <= limit;
+  std::printf("%s layers nq=%d dtype=%d segments=%d of at most %d\n", pass ? "ok" : "FAIL", nq, dtype, g_segments,
+              limit);
+  return pass ? 0 : 1;
+}
+
 int main() {
   std::mt19937_64 rng(20250117);
   int bad = 0;
@@ -316,5 +371,7 @@ int main() {
         bad += check<double>(rng, 4, true, 2, 4, count, mix, tail, from, 1e-10);
         bad += check<double>(rng, 5, true, 3, 5, count, mix, tail, from, 1e-10);
       }
+  for (int nq : {12, 13, 14}) bad += layers(nq, QJ_COMPLEX128, 5, 3);
+  for (int nq : {13, 14}) bad += layers(nq, QJ_COMPLEX64, 6, 4);
   return bad ? 1 : 0;
 }

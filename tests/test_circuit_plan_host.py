@@ -22,5 +22,5 @@ def test_planned_passes_equal_the_gates_in_order(tmp_path):
     proc = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     lines = proc.stdout.strip().splitlines()
     assert proc.returncode == 0, "\n".join(line for line in lines if not line.startswith("ok "))[-2000:]
-    assert len(lines) == 8 * 3 * 3 * 7
+    assert len(lines) == 8 * 3 * 3 * 7 + 5
     assert sum("permuted=1" in line for line in lines) > 20  # starts read permuted among them
