@@ -257,85 +257,156 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // Many outcomes (2^k > 32): a workgroup owns one value of the measured bits
-// above the row (bits >= LB, a row = kBlock x V consecutive amplitudes) and
+// above the row (bits >= lb, a row = kBlock x V consecutive amplitudes) and
 // walks a chunk of the free bits there, so every load of it is one whole row
 // and a thread keeps V sums; after the walk the row's free bits are summed in
 // LDS (a fixed tree) and its measured bits give the outcomes' low part.
-// Bound by the one read of the state.  The former kernel gave every thread an
-// outcome of its own and walked that outcome's amplitudes, one scattered
-// 16-byte load at a time: 10 of 28 qubits complex128 4.32 ms (1.0 TB/s),
-// now 0.81 ms (5.3 TB/s).
+// Where a value has few rows it owns B = 8 values: those of the three bits above
+// the row that are lowest in the outcome.  Their rows' loads are in flight
+// together, one set of barriers serves them all, and the outcomes are written in
+// ascending order, in runs of 8 also where the order of the qubits is reversed.
+// Bound by the one read of the state and the outcomes' stores.  28 qubits
+// complex128, against the kernel with a thread per outcome that walks the
+// outcome's amplitudes, one scattered 16-byte load at a time: all measured 3.21 ->
+// 1.16 ms (5.5 TB/s), in reversed order 9.26 -> 1.81, the first 26 1.67 -> 0.91, the
+// first 16 4.49 -> 0.69 (6.3 TB/s).  One value at a time: 3.93, 13.4, 4.06, 1.33.
 constexpr int kRowMaxBits = 9;
+constexpr int kRowBatchBits = 3;
+constexpr int kRowDirectBits = 3;  // free row bits that an outcome's thread sums by itself
+constexpr unsigned char kNoBit = 63;  // of an index that has fewer bits
 struct RowSpec {
-  int lb;                      // row bits
-  int nlow, low_bit[kRowMaxBits], low_out[kRowMaxBits];  // measured row bits -> outcome bits
-  int high_out[kMaxPos];       // measured bit j above the row -> outcome bit
-  Ins high;                    // measured bits above the row, relative to bit lb
-  unsigned free_mask;          // free row bits
+  int lb;                            // row bits
+  // amplitude bit -> bit of the item index, outcome bit -> bit of the item index,
+  // amplitude bit -> bit of the free rows' index (kNoBit: none)
+  unsigned char off_of[64], bin_of[64], free_of[64];
+  u64 batch_off[1 << kRowBatchBits];  // offsets of the item's rows
+  int nloc;                          // measured row and batch bits by ascending outcome bit,
+  u64 loc[2], loc_out[2];            // eight a word: LDS index bit, outcome bit
+  unsigned free_mask;                // free row bits
+  int nlast, last[kRowDirectBits];   // the lowest of them
 };
 
-template <typename R, typename T, int V>
+// Index bits moved to places: lane p holds where bit p comes from.  (Loops over
+// lists of positions, with a scalar load each, bound the kernel: 28 qubits
+// complex128, 25 of them measured, 1.79 ms.)
+__device__ __forceinline__ u64 place_bits(u64 index, int from) { return __ballot((int)((index >> from) & 1)); }
+
+// LDS slot of element e (row bits, then batch bits): the bits from 5 up are folded
+// into the bank, since an order of qubits may put them on the lanes.
+__device__ __forceinline__ unsigned row_slot(unsigned e) { return e ^ ((e >> 5) & 31u) ^ (e >> 10); }
+
+// Sum of the elements that differ from e in the row's lowest free bits, the
+// highest of them first (the order of the tree above it).
+template <int N>
+__device__ __forceinline__ double row_sum_of(const double* red, unsigned e, const int (&last)[kRowDirectBits]) {
+  double x[1 << N];
+#pragma unroll
+  for (int i = 0; i < (1 << N); ++i) {
+    unsigned m = e;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if ((i >> k) & 1) m |= 1u << last[k];
+    x[i] = red[row_slot(m)];
+  }
+#pragma unroll
+  for (int k = N - 1; k >= 0; --k)
+#pragma unroll
+    for (int i = 0; i < (1 << k); ++i) x[i] += x[i | (1 << k)];
+  return x[0];
+}
+__device__ __forceinline__ double row_sum(const double* red, unsigned e, int n, const int (&last)[kRowDirectBits]) {
+  switch (n) {  // uniform
+    case 0: return red[row_slot(e)];
+    case 1: return row_sum_of<1>(red, e, last);
+    case 2: return row_sum_of<2>(red, e, last);
+    default: return row_sum_of<3>(red, e, last);
+  }
+}
+
+template <typename R, typename T, int V, int BB>
 __global__ void __launch_bounds__(kBlock)
     k_probs_rows(const cplx<R>* __restrict__ st, u64 nitems, int chunk_bits, u64 per, u64 dstride, RowSpec rs,
                  double* __restrict__ partials, T* __restrict__ out) {
-  __shared__ double red[kBlock * V];
-  const unsigned row = 1u << rs.lb;
+  constexpr int B = 1 << BB;
+  __shared__ double red[B * kBlock * V];
+  const unsigned row = 1u << rs.lb, total = row << BB;
   const unsigned t = threadIdx.x * V;
+  const int lane = threadIdx.x & 63;
+  const int off_of = rs.off_of[lane], bin_of = rs.bin_of[lane], free_of = rs.free_of[lane];
+  // LDS element and outcome part of the local bits lo .. lo + 7 of an index
+  auto local = [&](unsigned i, int word, unsigned* e, u64* bin) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      *e |= ((i >> k) & 1u) << ((rs.loc[word] >> (8 * k)) & 31);
+      *bin |= (u64)((i >> k) & 1u) << ((rs.loc_out[word] >> (8 * k)) & 63);
+    }
+  };
+  unsigned my_e = 0;
+  u64 my_bin = 0;
+  local(threadIdx.x & ((1u << rs.nloc) - 1), 0, &my_e, &my_bin);
   for (u64 w = blockIdx.x; w < nitems; w += gridDim.x) {  // uniform per workgroup
     const u64 h = w >> chunk_bits, c = w & ((u64(1) << chunk_bits) - 1);
-    u64 off = 0, bin_high = 0;
-    for (int j = 0; j < rs.high.npos; ++j)
-      if ((h >> j) & 1) {
-        off |= u64(1) << rs.high.pos[j];
-        bin_high |= u64(1) << rs.high_out[j];
-      }
-    double acc[V];
+    const u64 off = place_bits(h, off_of), bin_high = place_bits(h, bin_of);
+    double acc[B][V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) acc[v] = 0.0;
+    for (int b = 0; b < B; ++b)
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[b][v] = 0.0;
     if (t < row) {
-      constexpr int U = 8;  // rows in flight
+      constexpr int U = BB ? 1 : 8;  // rows in flight beside the batch's
       for (u64 g = c * per; g < (c + 1) * per; g += U) {
         const int cnt = (c + 1) * per - g < U ? (int)((c + 1) * per - g) : U;
         if (dstride) {
           for (int u = 0; u < cnt; ++u)
 #pragma unroll
-            for (int v = 0; v < V; ++v)
-              acc[v] += prob_at(st, ((insert_bits(g + u, rs.high) | off) << rs.lb) + t + v, dstride);
-        } else if (cnt == U) {
-          cvec<R, V> x[U];
+            for (int b = 0; b < B; ++b)
 #pragma unroll
-          for (int u = 0; u < U; ++u) x[u] = ldv<R, V>(st + ((insert_bits(g + u, rs.high) | off) << rs.lb) + t);
+              for (int v = 0; v < V; ++v)
+                acc[b][v] += prob_at(st, (place_bits(g + u, free_of) | off | rs.batch_off[b]) + t + v,
+                                     dstride);
+        } else if (cnt == U) {
+          cvec<R, V> x[U][B];
 #pragma unroll
           for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int v = 0; v < V; ++v) acc[v] += abs2(x[u].v[v]);
+            for (int b = 0; b < B; ++b)
+              x[u][b] = ldv<R, V>(st + (place_bits(g + u, free_of) | off | rs.batch_off[b]) + t);
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int b = 0; b < B; ++b)
+#pragma unroll
+              for (int v = 0; v < V; ++v) acc[b][v] += abs2(x[u][b].v[v]);
         } else {
           for (int u = 0; u < cnt; ++u) {
-            const cvec<R, V> x = ldv<R, V>(st + ((insert_bits(g + u, rs.high) | off) << rs.lb) + t);
+            const cvec<R, V> x = ldv<R, V>(st + (place_bits(g + u, free_of) | off) + t);
 #pragma unroll
-            for (int v = 0; v < V; ++v) acc[v] += abs2(x.v[v]);
+            for (int v = 0; v < V; ++v) acc[0][v] += abs2(x.v[v]);  // U > 1: no batch
           }
         }
       }
-    }
 #pragma unroll
-    for (int v = 0; v < V; ++v) red[t + v] = acc[v];
+      for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int v = 0; v < V; ++v) red[row_slot((b << rs.lb) + t + v)] = acc[b][v];
+    }
     __syncthreads();
     unsigned done = 0;
-    for (unsigned rest = rs.free_mask; rest;) {  // uniform: highest free row bit first
+    for (unsigned rest = rs.free_mask; __popc(rest) > kRowDirectBits;) {  // uniform: highest free row bit first
       const unsigned bit = 1u << (31 - __clz(rest));
       rest ^= bit;
       done |= bit;
-      for (unsigned e = threadIdx.x; e < row; e += kBlock)
-        if (!(e & done)) red[e] += red[e | bit];
+      for (unsigned e = threadIdx.x; e < total; e += kBlock)
+        if (!(e & done)) red[row_slot(e)] += red[row_slot(e | bit)];
       __syncthreads();
     }
-    for (unsigned e = threadIdx.x; e < row; e += kBlock) {
-      if (e & rs.free_mask) continue;
-      u64 bin = bin_high;
-      for (int j = 0; j < rs.nlow; ++j) bin |= (u64)((e >> rs.low_bit[j]) & 1) << rs.low_out[j];
-      if (chunk_bits == 0) out[bin] = (T)red[e];
-      else partials[(bin << chunk_bits) + c] = red[e];
+    for (unsigned i = threadIdx.x; i < (1u << rs.nloc); i += kBlock) {
+      unsigned e = my_e;
+      u64 bin = bin_high | my_bin;
+      if (i >= 256) local(i >> 8, 1, &e, &bin);
+      const double x = row_sum(red, e, rs.nlast, rs.last);
+      if (chunk_bits == 0) out[bin] = (T)x;
+      else partials[(bin << chunk_bits) + c] = x;
     }
     __syncthreads();
   }
@@ -839,36 +910,68 @@ static int probs_impl(const void* state, int nqubits, const int32_t* qubits, int
   std::memset(&rs, 0, sizeof(rs));
   rs.lb = std::min(nqubits, pair ? kRowMaxBits : kRowMaxBits - 1);
   rs.free_mask = (1u << rs.lb) - 1;
-  for (int j = 0; j < nm; ++j) {  // ascending measured bits
-    int o = 0;                    // outcome bit of this position
-    while (obits.pos[nm - 1 - o] != sorted[j]) ++o;
-    if (sorted[j] < rs.lb) {
-      rs.low_bit[rs.nlow] = sorted[j];
-      rs.low_out[rs.nlow++] = o;
-      rs.free_mask &= ~(1u << sorted[j]);
-    } else {
-      rs.high_out[rs.high.npos] = o;
-      rs.high.pos[rs.high.npos++] = sorted[j] - rs.lb;
-    }
+  int out_of[kMaxPos], nhigh = 0;  // outcome bit of the measured bit sorted[j]
+  for (int j = 0; j < nm; ++j) {
+    out_of[j] = 0;
+    while (obits.pos[nm - 1 - out_of[j]] != sorted[j]) ++out_of[j];
+    if (sorted[j] < rs.lb) rs.free_mask &= ~(1u << sorted[j]);
+    else ++nhigh;
   }
-  // the free rows of an outcome are split until the launch has 32 workgroups
-  // per CU (kProbsMaxBlocks); the partials then hold 2^nlow sums of each, at
-  // most 2^9 x 2^13
-  const int free_bits = nqubits - rs.lb - rs.high.npos;
+  for (int b = 0; b < rs.lb && rs.nlast < kRowDirectBits; ++b)
+    if ((rs.free_mask >> b) & 1) rs.last[rs.nlast++] = b;
+  // The free rows of an outcome are split, down to 16 (two groups of loads; less
+  // would not pay for the launch that adds the partial sums: 10 to 12 qubits 16 us
+  // instead of 11), until the launch has a workgroup per CU, and on to 32
+  // (kProbsMaxBlocks) while the partial sums stay below 1/32 of the state's
+  // numbers (20 qubits, 15 measured, complex128: 40 us with 2^20 partials, 18
+  // without).
+  const int free_bits = nqubits - rs.lb - nhigh;
   int chunk_bits = 0;
-  while (chunk_bits < free_bits && (u64(1) << (rs.high.npos + chunk_bits)) < kProbsMaxBlocks &&
-         (nbins << (chunk_bits + 1)) <= sc->partials_cap)
+  while (free_bits - chunk_bits > 4 && (u64(1) << (nhigh + chunk_bits)) < kProbsMaxBlocks &&
+         (nbins << (chunk_bits + 1)) <= sc->partials_cap &&
+         (nhigh + chunk_bits < 8 || (nbins << (chunk_bits + 6)) <= (u64(1) << nqubits)))
     ++chunk_bits;
-  const u64 nitems = u64(1) << (rs.high.npos + chunk_bits), per = u64(1) << (free_bits - chunk_bits);
+  // Eight rows at a time where a value has fewer than eight to load and 512
+  // workgroups remain (20 qubits, all measured: 19 us without, 11 with).
+  const bool batch = dstride == 0 && nhigh >= kRowBatchBits && free_bits - chunk_bits < 3 && nhigh + chunk_bits >= 12;
+  const int nbatch = batch ? kRowBatchBits : 0;
+  std::memset(rs.off_of, kNoBit, sizeof(rs.off_of));
+  std::memset(rs.bin_of, kNoBit, sizeof(rs.bin_of));
+  std::memset(rs.free_of, kNoBit, sizeof(rs.free_of));
+  int nitem = 0;
+  auto add_local = [&](int index_bit, int o) {
+    rs.loc[rs.nloc / 8] |= (u64)index_bit << (8 * (rs.nloc % 8));
+    rs.loc_out[rs.nloc / 8] |= (u64)o << (8 * (rs.nloc % 8));
+    ++rs.nloc;
+  };
+  for (int o = 0, taken = 0; o < nm; ++o)  // ascending outcome bits
+    for (int j = 0; j < nm; ++j) {
+      if (out_of[j] != o) continue;
+      if (sorted[j] < rs.lb) {
+        add_local(sorted[j], o);
+      } else if (taken < nbatch) {
+        for (int b = 0; b < (1 << kRowBatchBits); ++b)
+          if ((b >> taken) & 1) rs.batch_off[b] |= u64(1) << sorted[j];
+        add_local(rs.lb + taken++, o);
+      } else {
+        rs.off_of[sorted[j]] = rs.bin_of[o] = (unsigned char)nitem++;
+      }
+    }
+  for (int b = rs.lb, f = 0; b < nqubits; ++b)
+    if (!std::binary_search(sorted.begin(), sorted.end(), b)) rs.free_of[b] = (unsigned char)f++;
+  const u64 nitems = u64(1) << (nitem + chunk_bits), per = u64(1) << (free_bits - chunk_bits);
   dim3 gd((unsigned)grid_for(nitems, 1)), bd(kBlock);
-  if (pair)
-    k_probs_rows<R, T, sizeof(R) == 4 ? 2 : 1><<<gd, bd, 0, s>>>(st, nitems, chunk_bits, per, dstride, rs,
-                                                                 sc->partials, out);
-  else
-    k_probs_rows<R, T, 1><<<gd, bd, 0, s>>>(st, nitems, chunk_bits, per, dstride, rs, sc->partials, out);
+  constexpr int VV = sizeof(R) == 4 ? 2 : 1;
+#define QJ_ROWS(V, BB) \
+  k_probs_rows<R, T, V, BB><<<gd, bd, 0, s>>>(st, nitems, chunk_bits, per, dstride, rs, sc->partials, out)
+  if (pair && batch) QJ_ROWS(VV, kRowBatchBits);
+  else if (pair) QJ_ROWS(VV, 0);
+  else if (batch) QJ_ROWS(1, kRowBatchBits);
+  else QJ_ROWS(1, 0);
+#undef QJ_ROWS
   rc = check_launch("probabilities launch");
   if (rc || chunk_bits == 0) return rc;
-  if (chunk_bits <= 4)
+  if (chunk_bits <= 4 || nm >= 15)  // a thread per outcome; otherwise a workgroup
     k_probs_finalize<T><<<dim3((unsigned)grid_for(nbins, kBlock)), dim3(kBlock), 0, s>>>(sc->partials, nbins,
                                                                                        chunk_bits, out);
   else

@@ -25,6 +25,25 @@ def test_marginal(backend, dtype, n, where):
     backend.set_dtype(dtype)
     qubits = {"high": [0, 1, 2, 3, 4, 5], "low": [n - 1, n - 2, n - 4, n - 5, n - 7, n - 8],
               "mixed": [n - 1, 3, n // 2, 0, n - 6, 7], "eleven": list(range(1, n, 2))[:11]}[where]
+    _check_marginal(backend, dtype, n, qubits)
+
+
+# eight rows at a time: free bits in the row (the lowest), above it and both, up
+# to three of them and more, outcomes in and against the order of the memory
+@pytest.mark.parametrize("n", [20, 21])
+@pytest.mark.parametrize("free", [[], [0], [19], [1, 18], [0, 1, 2], [17, 18, 19], [16, 17, 18, 19], [2, 9, 12, 16, 19]])
+@pytest.mark.parametrize("order", ["sorted", "reversed", "shuffled"])
+def test_nearly_all_measured(backend, dtype, n, free, order, rng):
+    backend.set_dtype(dtype)
+    qubits = [q for q in range(n) if q not in free]
+    if order == "reversed":
+        qubits.reverse()
+    elif order == "shuffled":
+        qubits = [int(q) for q in rng.permutation(qubits)]
+    _check_marginal(backend, dtype, n, qubits)
+
+
+def _check_marginal(backend, dtype, n, qubits):
     state = _random_state(n, dtype)
     got = backend.calculate_probabilities(state, qubits, n).double()
     probs = torch.view_as_real(state).double().square().sum(-1)
