@@ -110,6 +110,7 @@ __device__ __forceinline__ void count_product(uint32_t mx, uint32_t mz, uint32_t
 
 struct RowsArgs {
   const uint32_t* tab;
+  uint32_t* out;          // not SYM: the tableau again where its one workgroup writes it, else null
   int64_t ws;
   int n, m, S;            // qubits, measured qubits, sign columns
   const int32_t* qubits;
@@ -125,6 +126,27 @@ struct RowsArgs {
   int32_t* nrandom;
 };
 
+// Word w of a tableau column from its destabilizer words de and stabilizer
+// words st (nw each): the latter start at bit n.  Bit 2n, the scratch row's, is
+// `sum`, or stays what it is in `old` unless it was `set`.
+__device__ __forceinline__ uint32_t merged_word(const uint32_t* de, const uint32_t* st, int nw, int n, int64_t w,
+                                                bool set, uint32_t sum, uint32_t old) {
+  uint32_t v = 0;
+  if (w < nw) v = de[w] & rows_below(w, n);
+  // stabilizer rows n + i, i = 32 w - n + bit
+  const int64_t i0 = w * 32 - n;
+  if (i0 > -32) {
+    uint64_t pair = 0;
+    const int64_t f = i0 >> 5;  // floor
+    if (f >= 0 && f < nw) pair = st[f];
+    if (f + 1 < nw) pair |= (uint64_t)st[f + 1] << 32;
+    v |= (uint32_t)(pair >> (i0 & 31)) & rows_below(w, 2 * (int64_t)n) & ~rows_below(w, n);
+  }
+  const int64_t s2 = 2 * (int64_t)n;
+  if (w == (s2 >> 5)) v |= (set ? sum : (old >> (s2 & 31)) & 1u) << (s2 & 31);
+  return v;
+}
+
 template <int R, bool SYM>
 __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a) {
   extern __shared__ uint32_t rows_lds[];
@@ -138,21 +160,32 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
   uint32_t* scr = rowp + a.dw;
   const int nchunk = (C + 63) >> 6;  // 2 * nchunk == dw
   {
+    // eight words of each half in flight per thread: a column's words are one
+    // stride of the tableau apart, so every load is a memory round trip
+    constexpr int U = 8;
     const int sh = n & 31;
-    for (int e = t; e < C * R; e += kRowsThreads) {
-      const int c = e / R, w = w0 + e % R;
-      uint32_t d = 0, v = 0;
-      if (c <= 2 * n && w < nw) {
-        const uint32_t* col = a.tab + (int64_t)c * a.ws;
-        const uint32_t mask = rows_below(w, n);
-        d = col[w] & mask;
-        const int64_t f = ((int64_t)n + (int64_t)w * 32) >> 5;  // bits n+32w .. n+32w+31 of the column
-        v = col[f] >> sh;
-        if (sh && f + 1 < a.ws) v |= col[f + 1] << (32 - sh);
-        v &= mask;
+    for (int e0 = t; e0 < C * R; e0 += U * kRowsThreads) {
+      uint32_t d[U], lo[U], hi[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * kRowsThreads, c = e / R, w = w0 + e % R;
+        d[u] = lo[u] = hi[u] = 0;
+        if (e < C * R && c <= 2 * n && w < nw) {
+          const uint32_t* col = a.tab + (int64_t)c * a.ws;
+          const int64_t f = ((int64_t)n + (int64_t)w * 32) >> 5;  // bits n+32w .. n+32w+31 of the column
+          d[u] = col[w];
+          lo[u] = col[f];
+          if (f + 1 < a.ws) hi[u] = col[f + 1];
+        }
       }
-      DE[e] = d;
-      ST[e] = v;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * kRowsThreads;
+        if (e >= C * R) break;
+        const uint32_t mask = rows_below(w0 + e % R, n);
+        DE[e] = d[u] & mask;
+        ST[e] = (uint32_t)((((uint64_t)hi[u] << 32) | lo[u]) >> sh) & mask;
+      }
     }
   }
   int count = 0;
@@ -370,7 +403,16 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
       if (!ok) break;   // uniform
     }
   }
-  if (!SYM) {
+  if (!SYM && a.out) {
+    const int64_t W = (2 * (int64_t)n + 1 + 31) / 32;
+    for (int64_t e = t; e < (2 * (int64_t)n + 1) * W; e += kRowsThreads) {
+      const int64_t c = e / W, w = e - c * W;
+      const int word = c == 2 * n ? 0 : (int)(c >> 5), sh = c == 2 * n ? 0 : (int)(c & 31);
+      const uint32_t sum = det_any ? (c == 2 * n ? scr_sign : scr[word] >> sh) & 1u : 0u;
+      uint32_t* p = a.out + c * a.ws + w;
+      *p = merged_word(DE + c * R, ST + c * R, R, n, w, det_any, sum, *p);
+    }
+  } else if (!SYM) {
     const int nwp = G * R;
     for (int e = t; e < (2 * n + 1) * R; e += kRowsThreads) {
       const int c = e / R, w = w0 + e % R;
@@ -386,7 +428,8 @@ __global__ __launch_bounds__(kRowsThreads) void k_cliff_measure_rows(RowsArgs a)
 }
 
 // Tableau words from the staged rows: thread per (column, word).  The scratch
-// row is the sum of the workgroups' partial rows, or stays what it was.
+// row is the sum of the workgroups' partial rows (eight loads of the chain at a
+// time: 188 partial rows, 6000 qubits, one by one took 100 us), or stays what it was.
 __global__ void k_cliff_merge_rows(uint32_t* __restrict__ tab, int n, int64_t ws, int64_t W, RowsArgs a, int G,
                                    int R) {
   const int64_t C = 2 * (int64_t)n + 1;
@@ -394,31 +437,23 @@ __global__ void k_cliff_merge_rows(uint32_t* __restrict__ tab, int n, int64_t ws
   if (e >= C * W) return;
   const int64_t c = e / W, w = e - c * W;
   const int nwp = G * R;
-  const uint32_t* de = a.stage + c * nwp;
-  const uint32_t* st = a.stage + (C + c) * nwp;
-  uint32_t v = 0;
-  if (w < nwp) v = de[w] & rows_below(w, n);
-  // stabilizer rows n + i, i = 32 w - n + bit
-  const int64_t i0 = w * 32 - n;
-  if (i0 > -32) {
-    uint64_t pair = 0;
-    const int64_t f = i0 >> 5;  // floor
-    if (f >= 0 && f < nwp) pair = st[f];
-    if (f + 1 < nwp) pair |= (uint64_t)st[f + 1] << 32;
-    v |= (uint32_t)(pair >> (i0 & 31)) & rows_below(w, 2 * (int64_t)n) & ~rows_below(w, n);
-  }
   const int64_t s2 = 2 * (int64_t)n;
-  if (w == (s2 >> 5)) {
-    uint32_t bit;
-    if (a.det_any[0]) {
-      uint32_t x = 0;
-      const int word = c == s2 ? a.dw : (int)(c >> 5), sh = c == s2 ? 0 : (int)(c & 31);
-      for (int g = 0; g < G; ++g) x ^= a.scratch[(size_t)g * (a.dw + 1) + word] >> sh;
-      bit = x & 1u;
-    } else {
-      bit = (tab[c * ws + w] >> (s2 & 31)) & 1u;
+  uint32_t sum = 0;
+  if (w == (s2 >> 5) && a.det_any[0]) {
+    constexpr int U = 8;
+    const int word = c == s2 ? a.dw : (int)(c >> 5), sh = c == s2 ? 0 : (int)(c & 31);
+    const uint32_t* p = a.scratch + word;
+    int g = 0;
+    for (; g + U <= G; g += U) {
+      uint32_t x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = p[(size_t)(g + u) * (a.dw + 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) sum ^= x[u];
     }
-    v |= bit << (s2 & 31);
+    for (; g < G; ++g) sum ^= p[(size_t)g * (a.dw + 1)];
+    sum = (sum >> sh) & 1u;
   }
-  tab[c * ws + w] = v;
+  uint32_t* out = tab + c * ws + w;
+  *out = merged_word(a.stage + c * nwp, a.stage + (C + c) * nwp, nwp, n, w, a.det_any[0], sum, *out);
 }

@@ -1459,7 +1459,10 @@ int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStr
   }
   const int64_t W = cliff_words(a.n), C = 2 * (int64_t)a.n + 1;
   const size_t posts = (size_t)2 * p.G * (1 + p.dw);
-  const size_t stage = SYM ? 0 : (size_t)2 * C * p.G * p.R, scratch = SYM ? 0 : (size_t)p.G * (p.dw + 1);
+  // up to 128 qubits the one workgroup writes the tableau itself (one qubit of 64:
+  // 34 us for the call, 37 with the merge's launch; 256 qubits 42 and 39)
+  const bool merge = !SYM && (p.G > 1 || p.R == 8);
+  const size_t stage = merge ? (size_t)2 * C * p.G * p.R : 0, scratch = merge ? (size_t)p.G * (p.dw + 1) : 0;
   // Work space behind the qubit list in its ring slot, which the slot's event
   // guards on every stream (up to about 700 qubits; always in the symbolic form
   // with a few thousand sign columns), else the device's scratch, as the
@@ -1485,6 +1488,7 @@ int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStr
     area = sc->big;
   }
   a.tab = tab;
+  a.out = merge ? nullptr : tab;
   a.ws = cliff_stride(a.n);
   a.dw = p.dw;
   a.hdr = static_cast<post_t*>(area);
@@ -1503,7 +1507,7 @@ int launch_measure_rows(uint32_t* tab, RowsArgs a, const int32_t* qubits, hipStr
     *rc = hip_status(hipLaunchCooperativeKernel(kern, dim3((unsigned)p.G), dim3(kRowsThreads), args,
                                                 (unsigned)p.lds, s), "clifford_measure cooperative launch");
   }
-  if (!*rc && !SYM) {
+  if (!*rc && merge) {
     k_cliff_merge_rows<<<dim3(blocks_for(C * W, kBlock)), dim3(kBlock), 0, s>>>(tab, a.n, a.ws, W, a, p.G, p.R);
     *rc = check_launch("clifford_measure merge launch");
   }
@@ -1700,7 +1704,12 @@ int qj_clifford_measure(uint32_t* tab, int nqubits, const int32_t* qubits, int m
   const char* mode = std::getenv("QJ_CLIFFORD_MEASURE");
   const bool force_kernels = mode && std::strcmp(mode, "kernels") == 0;
   const bool force_small = mode && std::strcmp(mode, "small") == 0;
-  if (!exact && !force_kernels && !force_small) {
+  // The one-launch loop takes and returns the whole tableau (65 us for a call on
+  // 1000 qubits, 80 on 2000, 145 to 170 on 6000, and 2 to 5 us a measured qubit);
+  // launches per qubit start at 50 us and take 20 (few rows to multiply) to 50
+  // (random Clifford states, 3000 qubits) us a qubit.
+  const bool rows = nqubits <= kMeasureSmallMax || 2500 * (int64_t)(m - 1) > nqubits;
+  if (rows && !exact && !force_kernels && !force_small) {
     RowsArgs a;
     std::memset(&a, 0, sizeof(a));
     a.n = nqubits;
