@@ -278,10 +278,15 @@ bool merge(Item& it, const Item& p) {
   return false;
 }
 
+// What an LDS-kernel pass may take: its ops and matrices travel in one slot of
+// the staging ring.  kLdsOthers: ops per one that needs the LDS kernel.
+constexpr size_t kLdsBudget = kRingSlotBytes / 2;
+constexpr int kLdsOthers = 8;
+
 // Appends an op to a pass: phases join the latest item they can merge with
 // while everything after it commutes with them.  False, and nothing is
 // changed, if the pass's plan would grow over its budget.
-bool add_item(std::vector<Item>& items, const GateOp& op, int esize, size_t* bytes) {
+bool add_item(std::vector<Item>& items, const GateOp& op, int esize, size_t* bytes, size_t budget) {
   Item it;
   it.op = op;
   if (op.kind == QJ_TILE_PHASE) {
@@ -291,7 +296,7 @@ bool add_item(std::vector<Item>& items, const GateOp& op, int esize, size_t* byt
         Item old = items[j];
         if (merge(items[j], it)) {
           const size_t now = *bytes - item_bytes(old, esize) + item_bytes(items[j], esize);
-          if (now > kPassBudget && now > *bytes) {
+          if (now > budget && now > *bytes) {
             items[j] = std::move(old);
             return false;
           }
@@ -303,7 +308,7 @@ bool add_item(std::vector<Item>& items, const GateOp& op, int esize, size_t* byt
     }
   }
   const size_t more = item_bytes(it, esize);
-  if (!items.empty() && more && *bytes + more > kPassBudget) return false;
+  if (!items.empty() && more && *bytes + more > budget) return false;
   *bytes += more;
   items.push_back(std::move(it));
   return true;
@@ -543,6 +548,17 @@ int run_pending(Run& run) {
   const int esize = (int)elem_size(run.dtype);
   const u64 low_mask = bit(std::min(run.low, run.nbits)) - 1;
   const u64 all = bit(run.nbits) - 1;
+  // A dense op too wide for the register kernel (complex128, five targets) fills
+  // its plan alone.  Where each tile has a CU to itself a pass that starts with
+  // one goes on with the LDS kernel: it takes more of them, which saves a pass
+  // and an upload each (16 of them on 16 qubits 1.88 -> 1.63 ms), and a few other
+  // ops between.  With many other ops, or more tiles, a pass of its own is faster
+  // (20 rotations each: 2.27 against 2.51 ms; 24 qubits: 9.8 against 17.8).
+  const u64 ntiles = u64(1) << (run.nbits - std::min(run.nbits, run.low + run.max_high));
+  const bool one_per_cu = tile_per_cu(ntiles);
+  auto wide = [&](const GateOp& op) {
+    return op.kind == QJ_TILE_DENSE && !tile_register_bits(run.dtype, op.k, ntiles);
+  };
   u64 first_high = fold_swaps(run, low_mask);
   Pending pend{run.ops, {}, 0};
   std::vector<int> keep;
@@ -570,6 +586,7 @@ int run_pending(Run& run) {
     }
     u64 high = first_high, bx = 0, bz = 0;
     size_t bytes = 0, i = 0;
+    int nwide = 0, nother = 0;  // of an LDS-kernel pass
     while (i < pend.size() && bx != all) {  // with every bit changed by an op left behind, none commutes
       const size_t nrun = swap_run(pend, i, &bits);
       const size_t n = nrun >= 2 ? nrun : 1;  // swaps of a run stay together
@@ -583,7 +600,13 @@ int run_pending(Run& run) {
       take = take && __builtin_popcountll(need) <= run.max_high;
       for (size_t j = i; j < i + n; ++j) {
         const GateOp& op = pend[j];
-        take = take && add_item(items, op, esize, &bytes);  // swaps take no room: a run is not cut
+        const bool lds = one_per_cu && (nwide || (items.empty() && wide(op)));
+        if (lds && op.kind != QJ_TILE_SWAP) {
+          if (wide(op)) nwide += take;
+          else take = take && ++nother <= kLdsOthers * nwide;
+        }
+        // swaps take no room: a run is not cut
+        take = take && add_item(items, op, esize, &bytes, lds ? kLdsBudget : kPassBudget);
         if (take) continue;
         bx |= op.X;
         bz |= op.Z;

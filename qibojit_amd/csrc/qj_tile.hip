@@ -706,17 +706,21 @@ static void device_limits(int* cus, size_t* max_lds) {
   *max_lds = dev >= 0 ? (size_t)mlds[dev] : 65536;
 }
 
+bool tile_per_cu(u64 ntiles) {
+  int cus = 0;
+  size_t max_lds = 0;
+  device_limits(&cus, &max_lds);
+  return ntiles <= (u64)cus;
+}
+
 int tile_register_bits(int dtype, int maxk, u64 ntiles) {
   const bool dbl = dtype == QJ_COMPLEX128;
   const char* kern = std::getenv("QJ_TILE_KERNEL");
   if (kern && std::strcmp(kern, "lds") == 0) return 0;
-  int cus = 0;
-  size_t max_lds = 0;
-  device_limits(&cus, &max_lds);
   const char* e = std::getenv("QJ_TILE_NRB");
   const int v = e ? std::atoi(e) : 0;
   const int lo = dbl ? 3 : 4, hi = dbl ? 4 : 5;
-  int nrb = (v >= lo && v <= hi) ? v : ntiles <= (u64)cus ? lo : 4;
+  int nrb = (v >= lo && v <= hi) ? v : tile_per_cu(ntiles) ? lo : 4;
   if (maxk > nrb) nrb = maxk;
   return nrb <= hi ? nrb : 0;
 }

@@ -45,6 +45,8 @@ namespace qj {
 // qubits or more 3%.  QJ_TILE_NRB overrides (4 or 5 for complex64, 3 or 4 for
 // complex128).
 int tile_register_bits(int dtype, int maxk, u64 ntiles);
+// Whether each of the tiles has a CU to itself.
+bool tile_per_cu(u64 ntiles);
 
 constexpr int kRegMaxSeg = 64;
 constexpr int kRegMaxBits = 16;

@@ -20,9 +20,10 @@ int set_error(int code, const char* fmt, ...) {
   return code;
 }
 // The rule of the launch (qj_tile.hip) on 256 CUs.
+bool tile_per_cu(u64 ntiles) { return ntiles <= 256; }
 int tile_register_bits(int dtype, int maxk, u64 ntiles) {
   const int most = dtype == QJ_COMPLEX128 ? 4 : 5;
-  const int bits = std::max(maxk, dtype == QJ_COMPLEX128 && ntiles <= 256 ? 3 : 4);
+  const int bits = std::max(maxk, dtype == QJ_COMPLEX128 && tile_per_cu(ntiles) ? 3 : 4);
   return bits <= most ? bits : 0;
 }
 }  // namespace qj
