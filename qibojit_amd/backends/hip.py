@@ -895,6 +895,8 @@ class HipBackend(Backend):
                     block, matrix = self._channel_superoperator(g)
                     if block is not None:
                         records.add_dense(DENSE_BITS, block + [q + nqubits for q in block], (), matrix)
+                        if records.count >= _RECORDS_PER_RUN:
+                            flush()
                         continue
                 # matrices are complex128 (exact phase angles), cast to the
                 # state's precision when a pass is encoded
