@@ -36,6 +36,7 @@
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "qj_common.h"
@@ -644,35 +645,39 @@ extern "C" int qj_run_gates(const void* source, int from_source, void* state, in
   if (low_bits < 1 || low_bits > nbits || max_high < 0 || low_bits + max_high > nbits ||
       low_bits + max_high > QJ_TILE_MAX_BITS)
     return set_error(QJ_EVALUE, "run_gates: bad tile (low_bits=%d, max_high=%d)", low_bits, max_high);
-  Run run;
-  run.source = source;
-  run.state = state;
-  run.dtype = dtype;
-  run.nbits = nbits;
-  run.low = low_bits;
-  run.max_high = max_high;
-  run.plan_only = state == nullptr;
-  run.from_source = from_source != 0;
-  run.stream = (hipStream_t)stream;
-  int64_t at = 0, par = 0;
-  while (at < nwords) {
-    if (nwords - at < 3) return set_error(QJ_EVALUE, "run_gates: truncated record");
-    const int code = recs[at], nt = recs[at + 1], nc = recs[at + 2];
-    if (code < 0 || code > QJ_GATE_LAST) return set_error(QJ_EVALUE, "run_gates: unknown gate code %d", code);
-    const bool dense = code == QJ_GATE_DENSE || code == QJ_GATE_DENSE_BITS;
-    const int want = code == QJ_GATE_SWAP ? 2 : 1;
-    if (nc < 0 || (dense ? (nt < 1 || nt > QJ_TILE_MAX_K) : nt != want) || nt + nc > nbits ||
-        (code == QJ_GATE_SWAP && nc) || nwords - at < 3 + (int64_t)nt + nc)
-      return set_error(QJ_EVALUE, "run_gates: bad record at word %lld", (long long)at);
-    const int64_t np = dense ? 2 * (int64_t(1) << (2 * nt)) : nparams_of(code);
-    if (nparams - par < np) return set_error(QJ_EVALUE, "run_gates: too few parameters");
-    const int rc = push_record(run, nqubits, density != 0, recs + at, params + par);
-    if (rc) return rc;
-    at += 3 + nt + nc;
-    par += np;
+  try {
+    Run run;
+    run.source = source;
+    run.state = state;
+    run.dtype = dtype;
+    run.nbits = nbits;
+    run.low = low_bits;
+    run.max_high = max_high;
+    run.plan_only = state == nullptr;
+    run.from_source = from_source != 0;
+    run.stream = (hipStream_t)stream;
+    int64_t at = 0, par = 0;
+    while (at < nwords) {
+      if (nwords - at < 3) return set_error(QJ_EVALUE, "run_gates: truncated record");
+      const int code = recs[at], nt = recs[at + 1], nc = recs[at + 2];
+      if (code < 0 || code > QJ_GATE_LAST) return set_error(QJ_EVALUE, "run_gates: unknown gate code %d", code);
+      const bool dense = code == QJ_GATE_DENSE || code == QJ_GATE_DENSE_BITS;
+      const int want = code == QJ_GATE_SWAP ? 2 : 1;
+      if (nc < 0 || (dense ? (nt < 1 || nt > QJ_TILE_MAX_K) : nt != want) || nt + nc > nbits ||
+          (code == QJ_GATE_SWAP && nc) || nwords - at < 3 + (int64_t)nt + nc)
+        return set_error(QJ_EVALUE, "run_gates: bad record at word %lld", (long long)at);
+      const int64_t np = dense ? 2 * (int64_t(1) << (2 * nt)) : nparams_of(code);
+      if (nparams - par < np) return set_error(QJ_EVALUE, "run_gates: too few parameters");
+      const int rc = push_record(run, nqubits, density != 0, recs + at, params + par);
+      if (rc) return rc;
+      at += 3 + nt + nc;
+      par += np;
+    }
+    int rc = run_pending(run);
+    if (!rc) rc = fill_state(run);  // no gates at all
+    if (npasses) *npasses = run.npasses;
+    return rc;
+  } catch (const std::bad_alloc&) {
+    return set_error(QJ_EMEMORY, "run_gates: out of host memory");
   }
-  int rc = run_pending(run);
-  if (!rc) rc = fill_state(run);  // no gates at all
-  if (npasses) *npasses = run.npasses;
-  return rc;
 }
