@@ -30,8 +30,9 @@
 // gates 0.82 instead of 0.68 ms.
 //
 // The same steps in Python, cutting the list in order, took about 8 us a gate,
-// more than the device needed: 20 qubits, 600 gates 5.3 -> 1.07 ms; the two-layer 26-qubit ansatz and its energy 5.9 -> 4.65 ms;
-// two layers of a noisy 12-qubit density matrix 1.83 -> 1.17 ms.
+// more than the device needed: 20 qubits, 600 gates 5.3 -> 1.07 ms; the two-layer
+// 26-qubit ansatz and its energy 5.9 -> 4.65 ms; two layers of a noisy 12-qubit
+// density matrix 1.83 -> 1.17 ms.
 #include <algorithm>
 #include <cmath>
 #include <complex>

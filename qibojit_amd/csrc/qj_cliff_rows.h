@@ -5,7 +5,7 @@
 // the same j, every column of them as R words each (the stabilizer words are
 // shifted so that both halves line up).  The row products of a random
 // outcome then need nothing from other rows but row p, and one measured
-// qubit costs one exchange between workgroups:
+// qubit costs two waits for other workgroups, one after the other:
 //  * every workgroup posts its first stabilizer row with x_q = 1 (the row's
 //    bits, gathered by ballots, and its index), or the parity of the
 //    selected stabilizer signs when it has none;
@@ -22,12 +22,13 @@
 // coefficient of the j-th random outcome (measurement_forms); the tableau is
 // not written back.
 //
-// What bounds it: a chain of m dependent steps, each one cross-XCD round trip
-// (about 2.5 us) and the update of a workgroup's slice in LDS.  The launch-per-
-// phase loop took 7-8 launches per qubit.  Per qubit: 2.9 us at 100 qubits (one
-// workgroup; 6.8 before), 4.4 at 1000 (32 workgroups; 26), 7.3 at 4000.  Two or
-// four words of rows per workgroup (fewer, larger) measured 8% and 40% slower
-// at 1000 qubits.
+// What bounds it: a chain of m dependent steps, each two cross-XCD round trips
+// (about 2.5 us together) and the update of a workgroup's slice in LDS.  The launch-
+// per-phase loop took 7-8 launches per qubit.  All qubits of a random Clifford
+// state, per qubit: 1.8 us at 100 qubits (one workgroup; 6.8 by columns), 3.3 at
+// 300, 4.25 at 1000 (32 workgroups; 26), 7.0 at 4000.  Two or four words of rows per
+// workgroup (fewer, larger) made a gate list and 1000 measured qubits 5.33 and 6.9
+// ms instead of 5.19.
 constexpr int kRowsMaxSpins = 1 << 22;
 
 typedef unsigned long long post_t;
