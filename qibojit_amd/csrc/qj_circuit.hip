@@ -69,7 +69,7 @@ struct Run {
   const void* source;
   void* state;
   int dtype, nbits, low, max_high;
-  bool from_source, plan_only;
+  bool from_source, plan_only, one_per_cu;
   hipStream_t stream;
   std::vector<c128> pool;
   std::vector<GateOp> ops;  // in circuit order
@@ -320,13 +320,13 @@ bool add_item(std::vector<Item>& items, const GateOp& op, int esize, size_t* byt
 // bits (each new register set re-lays the tile out through LDS);
 // the first run avoids the six lowest tile bits, which the loads keep on
 // the lanes of a wave.
-void order_items(std::vector<Item>& items, u64 lane_bits, int dtype, u64 ntiles) {
+void order_items(std::vector<Item>& items, u64 lane_bits, int dtype, bool one_per_cu) {
   int maxk = 0;
   for (const Item& it : items) {
     if (it.op.kind == QJ_TILE_SWAP) return;  // swaps relabel bits on the way
     if (it.op.kind == QJ_TILE_DENSE) maxk = std::max(maxk, it.op.k);
   }
-  const int nrb = tile_register_bits(dtype, maxk, ntiles);
+  const int nrb = tile_register_bits(dtype, maxk, one_per_cu);
   if (!nrb) return;  // the LDS kernel keeps no bits in registers
   std::vector<Item> out;
   out.reserve(items.size());
@@ -390,7 +390,7 @@ int emit_tile(Run& run, std::vector<Item>& items, u64 high) {
     lane_bits |= bit(sb);
     ++lanes;
   }
-  order_items(items, lane_bits, run.dtype, u64(1) << nout);
+  order_items(items, lane_bits, run.dtype, run.one_per_cu);
 
   std::vector<qj_tile_op> ops;
   std::vector<char> data;
@@ -556,10 +556,9 @@ int run_pending(Run& run) {
   // and an upload each (16 of them on 16 qubits 1.88 -> 1.63 ms), and a few other
   // ops between.  With many other ops, or more tiles, a pass of its own is faster
   // (20 rotations each: 2.27 against 2.51 ms; 24 qubits: 9.8 against 17.8).
-  const u64 ntiles = u64(1) << (run.nbits - std::min(run.nbits, run.low + run.max_high));
-  const bool one_per_cu = tile_per_cu(ntiles);
+  run.one_per_cu = tile_per_cu(u64(1) << (run.nbits - std::min(run.nbits, run.low + run.max_high)));
   auto wide = [&](const GateOp& op) {
-    return op.kind == QJ_TILE_DENSE && !tile_register_bits(run.dtype, op.k, ntiles);
+    return op.kind == QJ_TILE_DENSE && !tile_register_bits(run.dtype, op.k, run.one_per_cu);
   };
   u64 first_high = fold_swaps(run, low_mask);
   Pending pend{run.ops, {}, 0};
@@ -602,7 +601,7 @@ int run_pending(Run& run) {
       take = take && __builtin_popcountll(need) <= run.max_high;
       for (size_t j = i; j < i + n; ++j) {
         const GateOp& op = pend[j];
-        const bool lds = one_per_cu && (nwide || (items.empty() && wide(op)));
+        const bool lds = run.one_per_cu && (nwide || (items.empty() && wide(op)));
         if (lds && op.kind != QJ_TILE_SWAP) {
           if (wide(op)) nwide += take;
           else take = take && ++nother <= kLdsOthers * nwide;

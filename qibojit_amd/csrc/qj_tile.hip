@@ -713,14 +713,14 @@ bool tile_per_cu(u64 ntiles) {
   return ntiles <= (u64)cus;
 }
 
-int tile_register_bits(int dtype, int maxk, u64 ntiles) {
+int tile_register_bits(int dtype, int maxk, bool one_per_cu) {
   const bool dbl = dtype == QJ_COMPLEX128;
   const char* kern = std::getenv("QJ_TILE_KERNEL");
   if (kern && std::strcmp(kern, "lds") == 0) return 0;
   const char* e = std::getenv("QJ_TILE_NRB");
   const int v = e ? std::atoi(e) : 0;
   const int lo = dbl ? 3 : 4, hi = dbl ? 4 : 5;
-  int nrb = (v >= lo && v <= hi) ? v : tile_per_cu(ntiles) ? lo : 4;
+  int nrb = (v >= lo && v <= hi) ? v : one_per_cu ? lo : 4;
   if (maxk > nrb) nrb = maxk;
   return nrb <= hi ? nrb : 0;
 }
@@ -843,7 +843,7 @@ static int tile_pass_impl(const void* source, const int32_t* source_bits, void* 
   int cus = 0;
   size_t max_lds = 0;
   device_limits(&cus, &max_lds);
-  const int nrb = tile_register_bits(sizeof(R) == 8 ? QJ_COMPLEX128 : QJ_COMPLEX64, maxk, ntiles);
+  const int nrb = tile_register_bits(sizeof(R) == 8 ? QJ_COMPLEX128 : QJ_COMPLEX64, maxk, ntiles <= (u64)cus);
   if (nrb) {
     RegPlanIn in;
     std::memset(&in, 0, sizeof(in));

@@ -33,8 +33,7 @@
 
 namespace qj {
 
-// Register bits per thread of a pass of `ntiles` tiles whose widest dense op has
-// maxk targets; 0 when it needs the LDS kernel.  The planner orders the ops of a
+// Register bits per thread of a pass whose widest dense op has maxk targets; 0 when it needs the LDS kernel.  The planner orders the ops of a
 // pass by the same count.  Four, or what the widest dense op needs; complex128
 // takes three where each tile has a CU to itself: eight waves a CU instead of
 // four hide more of the re-layouts' latency than the extra ones cost.  12 to 20
@@ -44,7 +43,7 @@ namespace qj {
 // matrix (16 tiles a CU) takes 6% longer, the 26-qubit ansatz 2.5% and QFTs of 24
 // qubits or more 3%.  QJ_TILE_NRB overrides (4 or 5 for complex64, 3 or 4 for
 // complex128).
-int tile_register_bits(int dtype, int maxk, u64 ntiles);
+int tile_register_bits(int dtype, int maxk, bool one_per_cu);
 // Whether each of the tiles has a CU to itself.
 bool tile_per_cu(u64 ntiles);
 

@@ -21,9 +21,9 @@ int set_error(int code, const char* fmt, ...) {
 }
 // The rule of the launch (qj_tile.hip) on 256 CUs.
 bool tile_per_cu(u64 ntiles) { return ntiles <= 256; }
-int tile_register_bits(int dtype, int maxk, u64 ntiles) {
+int tile_register_bits(int dtype, int maxk, bool one_per_cu) {
   const int most = dtype == QJ_COMPLEX128 ? 4 : 5;
-  const int bits = std::max(maxk, dtype == QJ_COMPLEX128 && tile_per_cu(ntiles) ? 3 : 4);
+  const int bits = std::max(maxk, dtype == QJ_COMPLEX128 && one_per_cu ? 3 : 4);
   return bits <= most ? bits : 0;
 }
 }  // namespace qj
@@ -39,7 +39,7 @@ static int segments(int dtype, int nq, int low, const int32_t* high, int nhigh, 
   RegPlanIn in;
   std::memset(&in, 0, sizeof(in));
   in.TB = low + nhigh;
-  in.NRB = tile_register_bits(dtype, maxk, u64(1) << (nq - in.TB));
+  in.NRB = tile_register_bits(dtype, maxk, tile_per_cu(u64(1) << (nq - in.TB)));
   if (!in.NRB) return 0;
   in.S = dtype == QJ_COMPLEX64 ? 5 : 4;
   in.esize = (int)elem_size(dtype);
