@@ -66,6 +66,7 @@ def _fused_layers(n, nlayers, params):
 
 
 STEP_BITS, STEP_TILE, STEP_WORDS = 10, 12, 19
+REGISTER_BITS = 5  # largest register group
 
 
 def step_passes(nbits, k, run):
@@ -88,8 +89,11 @@ def step_passes(nbits, k, run):
 def _passes(n, k, tdtype):
     if k is None:
         return tile_passes(n)
+    groups = register_passes(n, k)
     if n < STEP_TILE:
-        return register_passes(n, k)
+        return groups
+    if max(len(ps.bits) for ps in groups) > REGISTER_BITS:
+        raise ValueError(f"Register groups hold at most {REGISTER_BITS} bits (got {k} for {n} qubits).")
     return step_passes(n, k, 4 if tdtype == torch.complex64 else 3)
 
 
